@@ -54,18 +54,17 @@ def parse():
 
 
 # FP32 work the compositor kernels execute per (pixel, Gaussian) pair, counted from their arithmetic
-# (fma two, add / mul / min / max / compare / exp / rcp one each; fixed tile origin): alpha evaluation
-# 42 for every evaluated pair (M rd 15, |grd|^2 5, capped reciprocal 2, grd x gro 9, its squared norm
-# 5, exponent scale 2, exp / opacity / clamp / threshold 4); forward composite 13 + 2 per colour
-# channel for every composited pair (hit distance 6, depth 2, transmittance and tests 5); backward
-# 72 + 4 per colour channel for every composited pair without ray gradients (hit distance and the
-# 1 / (1 - alpha) transmittance 10, dL/dalpha 6, the collapsed alpha and hit vectors 21, mean
-# gradient 7 (the lane's M^T product shared by its four pixels), the symmetric M gradient from the
-# ray offset 24, opacity and buffer 4). Evaluated and composited counts come from the kernels
-# themselves (pair_counts), so pairs skipped unevaluated by the culling are not counted.
-FLOPS_EVAL = 42
-FLOPS_FWD_CONTRIB = 13          # + 2 per colour channel
-FLOPS_BWD_CONTRIB = 72          # + 4 per colour channel
+# (fma two, add / mul / min / compare / exp / rcp one each) for tiles whose rays share one origin, as every
+# configuration's here do: alpha evaluation 25 for every evaluated pair (three affine forms 12, two squared
+# norms 6, reciprocal, exponent 2, exp, opacity / clamp / threshold 3); forward composite 10 + 2 per colour
+# channel for every composited pair (hit distance 2, depth 2, transmittance and tests 6); backward
+# 53 + 4 per colour channel for every composited pair without ray gradients (hit distance and the ray's
+# offset 5, the transmittance 4, dL/dalpha 8, the hit's 2, dL/dgro 12, its symmetric M gradient 21,
+# opacity 1). Evaluated and composited counts come from the kernels themselves (pair_counts), so pairs
+# skipped unevaluated by the culling are not counted.
+FLOPS_EVAL = 25
+FLOPS_FWD_CONTRIB = 10          # + 2 per colour channel
+FLOPS_BWD_CONTRIB = 53          # + 4 per colour channel
 # MI355X's published FP32 peak: 1024 SIMDs issue a wave64 FMA every 2 cycles at 2.4 GHz. The kernels
 # are also priced against the FMA rate this GPU measurably sustains (valu_ceiling), which runs below it
 # because the clock drops under a full VALU load.

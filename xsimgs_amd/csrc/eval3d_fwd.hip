@@ -54,8 +54,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     constexpr bool OP_IN_COL = CL > 0 && (CL & 3) != 0;
     // Every per-Gaussian slot is an array indexed by the batch position, so that one address register (16
     // times the position) serves all reads of a Gaussian; position NT holds a Gaussian no pixel takes,
-    // which fills the lists up to whole steps. The M rows' fourth components hold gro = M (o - mu) when
-    // the tile's rays share one origin, else the mean.
+    // which fills the lists up to whole steps. One origin: the affine rows with -log2(e) / 2 D^2, D and the
+    // opacity in the fourth components; else the rows of M with the mean there.
     __shared__ float4 s_m0[NT + 1], s_m1[NT + 1], s_m2[NT + 1];
     __shared__ float4 s_op[OP_IN_COL ? 1 : NT + 1];  // opacity, when no colour slot has room
     __shared__ float4 s_vel[DYN ? NT + 1 : 1];
@@ -63,6 +63,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     __shared__ int32_t s_id[CL > 0 || CDIM == 0 ? 1 : NT + 1];
     __shared__ float4 s_box[NS];                        // the strips' boxes of (x, y)
     __shared__ float s_ik[DYN ? 1 : PX][DYN ? 1 : NT];  // rays of one origin: each pixel's 1 / k
+    __shared__ TileFrame s_frame;
     __shared__ float s_slack[2][NW];  // largest distance from the first pixel's origin, and time from its own
     // [wavefront][staging wavefront]: the Gaussians it evaluates, and their number
     __shared__ uint16_t s_list[NW][NW][64 + 2 * U];
@@ -137,11 +138,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     // the tile's first pixel (always inside the image), its middle one and the left end of that one's row
     const int64_t p0 = (int64_t)cam * hw + (int64_t)trow * g.tile_h * g.width + tcol * g.tile_w;
     const int64_t ps = p0 + (int64_t)min(g.tile_h / 2, g.height - 1 - trow * g.tile_h) * g.width;
-    const f3 o0 = uniform3(ld3(p.ray_o + 3 * p0));
+    const f3 o0 = first_origin(ld3(p.ray_o + 3 * p0));
     float rt0 = 0.f;
-    if constexpr (DYN) rt0 = p.rtd ? uniform_f(p.rtd[p0]) : 0.f;
+    if constexpr (DYN) rt0 = p.rtd ? first_time(p.rtd[p0]) : 0.f;
     const TileBasis basis = uniform_basis(
         tile_basis(ld3(p.ray_d + 3 * (ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w))), ld3(p.ray_d + 3 * ps)));
+    if (tr == 0) put_basis(s_frame, basis);
     bool narrow = true, same = true;
     float far2 = 0.f, late = 0.f;
 #pragma unroll
@@ -178,18 +180,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     // one origin (as float32 values) and ordinary rays: the pairs in the turned frame's affine form
     const bool fixed = !DYN && kind == 3;
     const bool cull = (kind & 1) != 0;
-    float hx = 0.f, hy = 0.f;  // the tile's largest |x| and |y|
-    float slack_o = 0.f, slack_t = 0.f;
-    for (int k = 0; k < nw * PX; ++k) {
-        const float4 box = s_box[k];
-        hx = fmaxf(hx, fabsf(box.x) + box.z);
-        hy = fmaxf(hy, fabsf(box.y) + box.w);
-    }
-    for (int k = 0; k < nw; ++k) {
-        slack_o = fmaxf(slack_o, s_slack[0][k]);
-        slack_t = fmaxf(slack_t, s_slack[1][k]);
-    }
-    slack_o = __builtin_amdgcn_sqrtf(slack_o);
+    if (tr == 0) tile_bounds(s_frame, s_box, nw * PX, s_slack[0], s_slack[1], nw);
+    __syncthreads();
 
     // A pixel takes a pair when alpha > thr: the largest float below 1/255 while the pixel is open, then
     // infinity (also outside the image).
@@ -235,20 +227,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
                 }
                 f3 at = mu;  // where the Gaussian is at the first pixel's time
                 if constexpr (DYN) at = mu + rt0 * vel;
-                const RayFrame f = ray_frame(r0, r1, r2, at, o0, basis);
+                const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
                 if constexpr (FIXED) {
                     s_m0[tr] = make_float4(f.a1.x, f.a1.y, f.a1.z, f.D * f.D * -0.72134752f);
                     s_m1[tr] = make_float4(f.a2.x, f.a2.y, f.a2.z, f.D);
                     s_m2[tr] = make_float4(f.au.x, f.au.y, f.au.z, op);
-                    cg = strip_cull(f, mu, sc, q, op, hx, hy, -1.f, 0.f);
+                    cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy, -1.f, 0.f);
                 } else {
+                    const f3 away = at - o0;
                     s_m0[tr] = make_float4(r0.x, r0.y, r0.z, mu.x);
                     s_m1[tr] = make_float4(r1.x, r1.y, r1.z, mu.y);
                     s_m2[tr] = make_float4(r2.x, r2.y, r2.z, mu.z);
                     if constexpr (!OP_IN_COL) s_op[tr].x = op;
-                    const f3 away = at - o0;
-                    cg = strip_cull(f, mu, sc, q, op, hx, hy,
-                                    slack_o + slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)),
+                    cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy,
+                                    s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)),
                                     __builtin_amdgcn_sqrtf(dot(away, away)));
                     cg.keep_all = cg.keep_all || !cull;
                 }

@@ -1,11 +1,10 @@
 // eval3d compositing kernels (reference csrc/rasterization/eval3d_{fwd,bwd}.cu, eval3d_dynamic_*.cu).
 //
-// One workgroup per (camera, tile); in the forward one thread per pixel (up to 1024 threads, 16
-// wave64s), in the backward two or four pixels per thread. Gaussians of the tile's depth-sorted list are staged in LDS in batches of one
-// per thread. Per staged Gaussian the LDS slot holds M = S^-1 R^T (three rows) and, when every ray
-// of the tile starts at the same origin (decided by a block vote, always true for a static pinhole
-// or spherical camera), gro = M (o - mu): the per-pair work then only maps the ray direction.
-// These are the values the reference computes per pair, so results do not depend on the path.
+// One workgroup per (camera, tile). The tile's pixels form strips of 64 consecutive ones (row-major); a
+// wavefront owns one or more whole strips, one pixel of each per lane. Gaussians of the tile's depth-sorted
+// list are staged in LDS in batches. Tiles whose rays start at one origin (decided by a block vote, always
+// true for a static pinhole, fisheye or spherical camera) work in a turned frame and affine ray coordinates
+// (below); the others with the rows of M = S^-1 R^T, as the reference does per pair.
 #pragma once
 #include "xsg_common.h"
 
@@ -13,7 +12,8 @@ namespace xsg {
 
 constexpr int kTileThreads = 256;
 constexpr int kMaxTilePixels = 1024;  // largest tile: the reference's 1024-thread workgroup limit
-constexpr int kColorLdsMax = 16;  // backward: colour channels staged in LDS; larger CDIM read from HBM
+constexpr int kBwdNoRayCdim = 16;    // backward: channels up to which per-pixel ray gradients can be left out
+constexpr int kBwdColorLdsMax = 33;  // backward: channels staged in LDS; larger CDIM read from HBM
 
 // The backward's variants of one group are compiled in one translation unit (eval3d_bwd_g<k>.hip).
 #define XSG_CDIM_GROUP0(X) X(0) X(1) X(2) X(3) X(4) X(5)
@@ -33,35 +33,6 @@ struct TileGrid {
     int64_t n;          // Gaussians (flatten id = cam * n + gaussian)
     int64_t n_isects;
 };
-
-struct PixelCtx {
-    int cam, tile, tr;
-    int i, j;
-    bool inside;
-    int64_t pix;          // index into [n_cams, H, W]
-    int32_t range_start, range_end;
-};
-
-XSG_DEV PixelCtx pixel_ctx(const TileGrid& g, const int32_t* __restrict__ offsets) {
-    PixelCtx c;
-    const int n_tiles = g.n_tiles_w * g.n_tiles_h;
-    const int nblocks = n_tiles * g.n_cams;
-    const int logical = xcd_tile((int)blockIdx.x, nblocks);
-    c.cam = logical / n_tiles;
-    c.tile = logical - c.cam * n_tiles;
-    c.tr = threadIdx.x;
-    const int ty = c.tr / g.tile_w, tx = c.tr - ty * g.tile_w;
-    const int trow = c.tile / g.n_tiles_w, tcol = c.tile - trow * g.n_tiles_w;
-    c.i = trow * g.tile_h + ty;  // utils.h:32-44
-    c.j = tcol * g.tile_w + tx;
-    c.inside = c.tr < g.tile_w * g.tile_h && c.i < g.height && c.j < g.width;
-    const int64_t hw = (int64_t)g.width * g.height;
-    c.pix = (int64_t)c.cam * hw + min((int64_t)c.i * g.width + c.j, hw - 1);
-    const int gt = c.cam * n_tiles + c.tile;  // utils.h:48-58
-    c.range_start = offsets[gt];
-    c.range_end = (gt == nblocks - 1) ? (int32_t)g.n_isects : offsets[gt + 1];
-    return c;
-}
 
 // Rows of M = S^-1 R^T from the raw quaternion (w, x, y, z) and activated scales: row i is column i
 // of R / s_i (utils.h:61-83 and eval3d_fwd.cu:92-107).
@@ -85,53 +56,12 @@ XSG_DEV f3 rows_tmul(f3 r0, f3 r1, f3 r2, f3 v) {  // M^T v
                r0.z * v.x + r1.z * v.y + r2.z * v.z);
 }
 
-// 1/sqrt(l) for l > 0, else 1: safe_normalize(v) (utils.h:85-88) is v * inv_len(|v|^2). The raw
-// v_rsq_f32 (1 ulp) replaces rsqrtf, whose denormal-range scaling costs five more instructions.
-XSG_DEV float inv_len(float l) { return l > 0.0f ? __builtin_amdgcn_rsqf(l) : 1.0f; }
-
-XSG_DEV f3 safe_normalize(f3 v) { return v * inv_len(dot(v, v)); }
-
-// safe_normalize_bwd (utils.h:198-206) with il = inv_len(|v|^2) already known
-XSG_DEV f3 safe_normalize_bwd_il(f3 v, float il, f3 d_out) {
-    return il * d_out - (il * il * il * dot(d_out, v)) * v;
-}
-
 // Hides a value's origin from the optimiser (which would turn sign masks back into compares and selects,
 // at twice the issue cycles of the integer operations).
 XSG_DEV int32_t opaque(int32_t v) {
     asm("" : "+v"(v));
     return v;
 }
-
-// ---------------------------------------------------------------------------------------------
-// Conservative (wavefront, Gaussian) culling.
-//
-// A pair adds nothing unless alpha = min(0.999, op exp(-d^2 / 2)) >= 1/255, d = |n x gro| being
-// the distance, in the Gaussian's normalised frame (x -> M x, M = S^-1 R^T, centre at 0), from the
-// centre to the pixel's ray line {gro + t n}. For a wavefront, every ray starts within rho of a
-// point c and points within angle theta of a unit axis a. In the normalised frame the origins lie
-// within rho / s_min of g0 = M (c - mu), and each direction M d is within theta' of M a, with
-//   sin theta' <= sin theta |Ma x Mb| / (|Ma| |Md|) <= sin theta (s_max / (s1 s2 s3)) /
-//                 (|Ma| (|Ma| cos theta - sin theta / s_min))
-// (d = cos phi a + sin phi b, (Ma) x (Mb) = det M M^-T (a x b), |M^-T| = s_max, |Mb| <= 1/s_min).
-// So d >= (|g0 x Ma| cos theta' - |g0 . Ma| sin theta') / |Ma| - rho / s_min. Independently, as
-// |M w| >= |w| / s_max, d >= dist(mu, line) / s_max >= (|v x a| cos theta - |v . a| sin theta - rho)
-// / s_max with v = mu - c, which stays tight for very flat Gaussians where theta' is large. When
-// either bound exceeds d_lim = sqrt(2 ln(255 op)) (plus a bound on the f32 error of the per-pair
-// d) no pixel of the wavefront can take the Gaussian: the pair would be evaluated and skipped by the alpha test, and
-// skipping it unevaluated changes no output. Pairs whose per-pair math could overflow or produce
-// NaN (non-finite inputs, degenerate scales or rays) are always kept, so they reach the alpha test
-// as in the reference.
-struct RayBundle {
-    float cx, cy, cz;    // centre of the ray origins
-    float ax, ay, az;    // unit axis
-    float cos_t, sin_t;  // bound on the angle between a ray and the axis
-    float rho;           // bound on |o_i - c|
-    float rt_max;        // bound on |time delta| (dynamic)
-    float rd_max;        // bound on |rd_i|
-    int mode;            // kBundleCull, kBundleKeepAll or kBundleEmpty
-};
-constexpr int kBundleCull = 0, kBundleKeepAll = 1, kBundleEmpty = 2;
 
 // Reductions over a full wavefront by DPP moves (rows of 16 lanes, then row 0's and rows 0-1's last lanes
 // broadcast up), whose result lane 63 holds and every lane returns: a lane exchange through the LDS unit
@@ -150,9 +80,6 @@ XSG_DEV float wave_reduce_f(float v, float identity, F&& f) {
 #undef XSG_STEP
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
-XSG_DEV float wave_sum_f(float v) {
-    return wave_reduce_f(v, 0.f, [](float a, float b) { return a + b; });
-}
 XSG_DEV float wave_max_f(float v) {
     return wave_reduce_f(v, -__builtin_inff(), [](float a, float b) { return fmaxf(a, b); });
 }
@@ -165,9 +92,6 @@ XSG_DEV uint64_t uniform_u64(uint64_t v) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
     return ((uint64_t)hi << 32) | lo;
-}
-XSG_DEV float lane_f(float v, int lane) {  // lane: wave-uniform
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 XSG_DEV float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 XSG_DEV bool finite3(f3 v) { return isfinite(v.x) && isfinite(v.y) && isfinite(v.z); }
@@ -192,7 +116,7 @@ XSG_DEV bool finite3(f3 v) { return isfinite(v.x) && isfinite(v.y) && isfinite(v
 // the ray's distance from the Gaussian of about an ulp of |gro|, as with the cross product: t.A, the pixel's
 // (x, y) and D are therefore summed in float64 (once per Gaussian and tile, or pixel), t.A with the
 // residual of t.(o - mu), which the turn leaves at rounding, taken out. Measured over Gaussians of
-// exp(-3 +- 0.7) at 2 to 80 from the origin, the root mean square error of exp(-d^2 / 2) is 1e-6 or less,
+// exp(-3 +- 0.7) at 2 to 80 from the origin, the root mean square error of exp(-d^2 / 2) is 1.0e-7,
 // against 9.7e-6 with the cross product in float32.
 struct d3 {
     double x, y, z;
@@ -242,7 +166,28 @@ XSG_DEV double uniform_d(double v) {
 }
 XSG_DEV d3 uniform_d3(d3 v) { return d3{uniform_d(v.x), uniform_d(v.y), uniform_d(v.z)}; }
 XSG_DEV TileBasis uniform_basis(TileBasis b) { return TileBasis{uniform_d3(b.a), uniform_d3(b.x), uniform_d3(b.y)}; }
+
+// What staging a Gaussian needs of the tile, kept in LDS between batches (as scalars it would cost the pair
+// loops eighteen registers and their spills).
+struct TileFrame {
+    double basis[9];
+    float hx, hy, slack_o, slack_t;
+};
+XSG_DEV void put_basis(TileFrame& f, const TileBasis& b) {
+    f.basis[0] = b.a.x; f.basis[1] = b.a.y; f.basis[2] = b.a.z;
+    f.basis[3] = b.x.x; f.basis[4] = b.x.y; f.basis[5] = b.x.z;
+    f.basis[6] = b.y.x; f.basis[7] = b.y.y; f.basis[8] = b.y.z;
+}
+XSG_DEV TileBasis get_basis(const TileFrame& f) {
+    const double* b = f.basis + opaque(0);
+    return TileBasis{d3{b[0], b[1], b[2]}, d3{b[3], b[4], b[5]}, d3{b[6], b[7], b[8]}};
+}
 XSG_DEV f3 uniform3(f3 v) { return mk3(uniform_f(v.x), uniform_f(v.y), uniform_f(v.z)); }
+
+// What a tile's pixels count their origins and times from: the first pixel's, or 0 where that is no number
+// (which must not reach the other pixels).
+XSG_DEV f3 first_origin(f3 o) { return uniform3(finite3(o) ? o : mk3(0.f, 0.f, 0.f)); }
+XSG_DEV float first_time(float t) { return uniform_f(isfinite(t) ? t : 0.f); }
 
 // A pixel's (x, y) and 1 / k; false where the ray does not run within 60 degrees of the axis.
 XSG_DEV bool ray_xy(const TileBasis& b, f3 d, float& x, float& y, float& inv_k) {
@@ -262,6 +207,20 @@ XSG_DEV float4 strip_box(bool inside, float x, float y) {
     const bool any = x0 <= x1;
     return make_float4(any ? 0.5f * (x0 + x1) : 0.f, any ? 0.5f * (y0 + y1) : 0.f,
                        any ? 0.500001f * (x1 - x0) + 1e-7f : -1.f, any ? 0.500001f * (y1 - y0) + 1e-7f : -1.f);
+}
+
+// The tile's largest |x| and |y| and its slack (strip_cull), from its strips' and wavefronts'.
+XSG_DEV void tile_bounds(TileFrame& f, const float4* boxes, int n_boxes, const float* far2, const float* late, int nw) {
+    float hx = 0.f, hy = 0.f, o = 0.f, t = 0.f;
+    for (int k = 0; k < n_boxes; ++k) {
+        hx = fmaxf(hx, fabsf(boxes[k].x) + boxes[k].z);
+        hy = fmaxf(hy, fabsf(boxes[k].y) + boxes[k].w);
+    }
+    for (int k = 0; k < nw; ++k) {
+        o = fmaxf(o, far2[k]);
+        t = fmaxf(t, late[k]);
+    }
+    f.hx = hx; f.hy = hy; f.slack_o = __builtin_amdgcn_sqrtf(o); f.slack_t = t;
 }
 
 // One Gaussian's turned frame (rows in world space) and its affine rows (value, d/dx, d/dy).
@@ -298,6 +257,36 @@ XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& ba
     f.au = mk3(dot(f.u, ba), dot(f.u, bx), dot(f.u, by));
     f.D = (float)dot64(to64(f.u), v64);
     return f;
+}
+
+// A vector and a symmetric matrix (upper triangle, row-major) of the turned frame, turned back into the
+// Gaussian's own normalised frame; the rows, mean and origin are those ray_frame was given.
+XSG_DEV void turn_back(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, f3& v, float (&Q)[6]) {
+    const f3 g = rows_mul(r0, r1, r2, o - mu);
+    const float ax = fabsf(g.x), ay = fabsf(g.y), az = fabsf(g.z);
+    const bool kx = ax >= ay && ax >= az, ky = !kx && ay >= az;
+    const float gk = kx ? g.x : ky ? g.y : g.z, ga = kx ? g.y : g.x, gb = (kx || ky) ? g.z : g.y;
+    const float D = __builtin_amdgcn_sqrtf(dot(g, g));
+    const float vk = gk + copysignf(D, gk);
+    const float den = D * (D + fabsf(gk));
+    const float beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;
+    const float s = -copysignf(1.0f, gk);  // u is s times the reflected row k
+    const f3 n = mk3(ga, gb, vk);
+    f3 w = mk3(v.x, v.y, s * v.z);
+    w = w - (beta * dot(n, w)) * n;  // in the order (a, b, k)
+    v = mk3(kx ? w.z : w.x, kx ? w.x : ky ? w.z : w.y, (kx || ky) ? w.y : w.z);
+    const float aa = Q[0], ab = Q[1], ak = s * Q[2], bb = Q[3], bk = s * Q[4], kk = Q[5];
+    const f3 y = beta * mk3(aa * n.x + ab * n.y + ak * n.z, ab * n.x + bb * n.y + bk * n.z, ak * n.x + bk * n.y + kk * n.z);
+    // n z^T + z n^T with z = y - beta (n . y) / 2 n
+    const f3 z = y - (0.5f * beta * dot(n, y)) * n;
+    const float raa = aa - 2.f * n.x * z.x, rab = ab - n.x * z.y - n.y * z.x, rak = ak - n.x * z.z - n.z * z.x;
+    const float rbb = bb - 2.f * n.y * z.y, rbk = bk - n.y * z.z - n.z * z.y, rkk = kk - 2.f * n.z * z.z;
+    Q[0] = kx ? rkk : raa;
+    Q[1] = kx || ky ? rak : rab;
+    Q[2] = kx ? rbk : ky ? rab : rak;
+    Q[3] = kx ? raa : ky ? rkk : rbb;
+    Q[4] = kx ? rab : rbk;
+    Q[5] = kx || ky ? rbb : rkk;
 }
 
 // alpha / opacity of one pair; a.w = -log2(e) / 2 D^2. |grd|^2 is at least 1e-36, so that a Gaussian without
@@ -384,124 +373,6 @@ XSG_DEV bool strip_keep(float4 box, const StripCull& c) {
     const bool out = n1 * n1 + n2 * n2 > c.rho2 * bu * bu || fabsf(box.x - c.xg) > box.z + c.ex ||
                      fabsf(box.y - c.yg) > box.w + c.ey;
     return box.z >= 0.f && !c.drop_all && (c.keep_all || !out);
-}
-
-// Bundle of the P pixels per lane of a full wavefront (all 64 lanes active). Pixels outside the
-// image do not count; one inside pixel with a degenerate ray turns culling off for the wavefront.
-template <int P>
-XSG_DEV RayBundle wave_bundle(const bool (&inside)[P], const f3 (&ro)[P], const f3 (&rd)[P],
-                              const float (&rt)[P]) {
-    RayBundle b;
-    bool irregular = false, any = false;
-    f3 dn[P], sum = mk3(0.f, 0.f, 0.f), first = mk3(0.f, 0.f, 0.f);
-    bool use[P];
-    float rd2 = 0.f, rtm = 0.f;
-#pragma unroll
-    for (int h = P - 1; h >= 0; --h) {
-        const float l = dot(rd[h], rd[h]);
-        const bool reg = l >= 1e-12f && l <= 1e12f && finite3(ro[h]) && isfinite(rt[h]);
-        irregular = irregular || (inside[h] && !reg);
-        use[h] = inside[h] && reg;
-        any = any || use[h];
-        dn[h] = sel3(use[h], rd[h] * __builtin_amdgcn_rsqf(l), mk3(0.f, 0.f, 0.f));
-        sum = sum + dn[h];
-        rd2 = use[h] ? fmaxf(rd2, l) : rd2;
-        rtm = use[h] ? fmaxf(rtm, fabsf(rt[h])) : rtm;
-        first = sel3(use[h], ro[h], first);  // the lowest usable pixel of the lane
-    }
-    const uint64_t any_mask = __ballot(any);
-    const bool irr = __ballot(irregular) != 0;
-    sum = mk3(wave_sum_f(sum.x), wave_sum_f(sum.y), wave_sum_f(sum.z));
-    const float sl = dot(sum, sum);
-    const f3 a = sum * (sl > 0.f ? __builtin_amdgcn_rsqf(sl) : 0.f);
-    float smax = 0.f, cmin = 1.f;
-#pragma unroll
-    for (int h = 0; h < P; ++h) {
-        const f3 x = cross(dn[h], a);
-        smax = use[h] ? fmaxf(smax, __builtin_amdgcn_sqrtf(dot(x, x))) : smax;
-        cmin = use[h] ? fminf(cmin, dot(dn[h], a)) : cmin;
-    }
-    smax = wave_max_f(smax);
-    cmin = wave_min_f(cmin);
-    const int src = any_mask ? (int)__builtin_ctzll(any_mask) : 0;
-    const f3 c = mk3(lane_f(first.x, src), lane_f(first.y, src), lane_f(first.z, src));
-    float rho = 0.f;
-#pragma unroll
-    for (int h = 0; h < P; ++h) {
-        const f3 u = ro[h] - c;
-        rho = use[h] ? fmaxf(rho, __builtin_amdgcn_sqrtf(dot(u, u))) : rho;
-    }
-    rho = wave_max_f(rho);
-    b.cx = c.x; b.cy = c.y; b.cz = c.z;
-    b.ax = a.x; b.ay = a.y; b.az = a.z;
-    b.sin_t = fminf(1.f, smax * 1.00001f + 1e-6f);
-    b.cos_t = __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - b.sin_t * b.sin_t));
-    b.rho = rho * 1.000001f;
-    b.rt_max = wave_max_f(rtm);
-    b.rd_max = __builtin_amdgcn_sqrtf(wave_max_f(rd2)) * 1.000001f;
-    // a bundle wider than 60 degrees is not worth bounding
-    b.mode = any_mask == 0 ? kBundleEmpty : ((irr || !(sl > 0.f) || !(cmin > 0.5f)) ? kBundleKeepAll : kBundleCull);
-    return b;
-}
-
-// Per-Gaussian part of the test, computed once per staged Gaussian.
-struct CullGauss {
-    f3 mu, r0, r1, r2;  // centre and rows of M
-    float inv_smin;     // 1 / s_min
-    float s_max;
-    float cone;         // s_max / (s1 s2 s3) = 1 / (product of the two smaller scales)
-    float s_min, d_lim, vel_len;
-    bool ok;            // finite inputs, scales in [1e-12, 1e9], a quaternion that normalises
-    bool op_low;        // op < 1/255: alpha never reaches the threshold
-};
-
-XSG_DEV CullGauss cull_gauss(f3 mu, f3 r0, f3 r1, f3 r2, f3 s, float4 q, float op, f3 vel) {
-    CullGauss g;
-    g.mu = mu; g.r0 = r0; g.r1 = r1; g.r2 = r2;
-    const float s_max = fmaxf(s.x, fmaxf(s.y, s.z));
-    g.s_max = s_max;
-    g.s_min = fminf(s.x, fminf(s.y, s.z));
-    g.inv_smin = 1.f / g.s_min;
-    g.cone = s_max / (s.x * s.y * s.z);
-    const float q2 = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
-    g.vel_len = __builtin_amdgcn_sqrtf(dot(vel, vel));
-    g.ok = finite3(mu) && g.s_min >= 1e-12f && s_max <= 1e9f && q2 >= 1e-30f && q2 <= 1e30f && isfinite(op) &&
-           isfinite(g.vel_len);
-    g.op_low = op < 1.f / 255.f;
-    // 2 ln(255 op) through log2; + 3e-3 covers the rounding of log, exp, the product and the compare
-    const float l2 = 2.f * 0.69314718f * __builtin_amdgcn_logf(fmaxf(255.f * op, 1.f));
-    g.d_lim = __builtin_amdgcn_sqrtf(fmaxf(0.f, l2)) * 1.0001f + 3e-3f;
-    return g;
-}
-
-// True unless no pixel of the bundle can take the Gaussian.
-template <bool DYN>
-XSG_DEV bool cull_keep(const RayBundle& b, const CullGauss& g) {
-    if (b.mode != kBundleCull) return b.mode == kBundleKeepAll;
-    const f3 v = mk3(b.cx, b.cy, b.cz) - g.mu, a = mk3(b.ax, b.ay, b.az);
-    const f3 g0 = rows_mul(g.r0, g.r1, g.r2, v);  // M (c - mu)
-    const f3 ma = rows_mul(g.r0, g.r1, g.r2, a);  // M a
-    const float ma_len = __builtin_amdgcn_sqrtf(dot(ma, ma));
-    const float shift = b.rho + (DYN ? b.rt_max * g.vel_len : 0.f);  // |o_i - c| + |mu(t) - mu|
-    const float Dr = __builtin_amdgcn_sqrtf(dot(v, v)) + shift;     // bound on |o_i - mu(t)|
-    const float L = Dr * g.inv_smin;                                 // bound on |gro| of every pair
-    // per-pair products stay below 1e18, so the alpha test sees finite values
-    const bool safe = g.s_min * g.s_min * 1e18f >= Dr * b.rd_max;
-    const float mc = ma_len * b.cos_t, ms = b.sin_t * g.inv_smin;
-    const bool narrow = mc - ms > 0.01f * mc;  // the direction bound below holds, to 1% cancellation
-    const float sin_tp = fminf(1.f, b.sin_t * g.cone / (ma_len * (mc - ms)) * 1.00001f + 1e-6f);
-    const float cos_tp = __builtin_amdgcn_sqrtf(fmaxf(0.f, 1.f - sin_tp * sin_tp));
-    const f3 x = cross(g0, ma);
-    const float lhs = (__builtin_amdgcn_sqrtf(dot(x, x)) * cos_tp - fabsf(dot(g0, ma)) * sin_tp) / ma_len;
-    // 2e-5 L bounds the f32 error of the per-pair d (about 17 ulp of |gro|) and of these tests
-    const float d_err = g.d_lim + 2e-5f * L;
-    const bool far_n = narrow && lhs > d_err + shift * g.inv_smin * 1.00001f;
-    // world-space bound (1e-5 Dr: this test's own rounding)
-    const f3 xw = cross(v, a);
-    const float lhs_w = __builtin_amdgcn_sqrtf(dot(xw, xw)) * b.cos_t - fabsf(dot(v, a)) * b.sin_t;
-    const bool far_w = lhs_w > d_err * g.s_max * 1.0001f + shift * 1.00001f + 1e-5f * Dr;
-    const bool skip = g.ok && safe && (g.op_low || far_n || far_w);
-    return !skip;
 }
 
 // Lane-to-lane moves inside rows of 16 lanes (DPP). `update_dpp` with all rows/banks enabled and
