@@ -7,6 +7,7 @@
 // coalesced per thread and is read directly. The backward writes every band of d_coeffs (zeros
 // above the used degree), d_positions without atomics, and per-block d_origin partials that a
 // second kernel sums in a fixed order.
+#include <initializer_list>
 #include <mutex>
 
 #include "xsg_common.h"
@@ -272,6 +273,210 @@ __global__ __launch_bounds__(kBlock) void sh_fwd_3kn_kernel(
     }
 }
 
+// [3, K, N] with V Gaussians per thread: every band row is read (and in the backward written) as V-wide
+// vectors, so that a wavefront keeps V times the bytes in flight. HBM-bound; backward alone, 1.5 M Gaussians
+// of degree 3: 143 -> 109 us (4.4 -> 5.8 TB/s), 300 k: 24 -> 20 us; but 400 k of degree 2 15 -> 17 us, so
+// coefficients of less than kVecBytes keep the one-per-thread kernel. The gradient rows bypass the caches
+// (written once, read later). Coefficients that with their gradients outgrow the 256 MB last-level cache
+// (kStreamBytes) are read past it as well (NT), in the forward too, which gains nothing else from vectors:
+// both passes over three such sets in turn 217 -> 164 us (170 without), 1 M of degree 4 251 -> 171 (178); at
+// 115 MB 76 us against 67. Needs n a multiple of V and arrays aligned to the vectors (vec_ok); other calls
+// take the one-per-thread kernels. The values are computed as there, in the same order; only d_origin's
+// partial sums group other Gaussians.
+constexpr int64_t kVecBytes = 48ll << 20, kStreamBytes = 192ll << 20;
+
+template <bool NT, class T>
+XSG_DEV T load_vec(const T* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
+template <int V>
+struct VecF {
+    typedef float type __attribute__((ext_vector_type(V)));
+};
+
+template <int V>
+XSG_DEV void load3v(const float* __restrict__ src, float (&v)[3 * V]) {
+    typedef typename VecF<V>::type vf;
+    const vf* p = reinterpret_cast<const vf*>(src);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const vf a = p[k];
+#pragma unroll
+        for (int j = 0; j < V; ++j) v[k * V + j] = a[j];
+    }
+}
+template <int V>
+XSG_DEV void store3v(float* __restrict__ dst, const float (&v)[3 * V]) {
+    typedef typename VecF<V>::type vf;
+    vf* p = reinterpret_cast<vf*>(dst);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        vf a;
+#pragma unroll
+        for (int j = 0; j < V; ++j) a[j] = v[k * V + j];
+        p[k] = a;
+    }
+}
+
+template <int DEG, bool HAS_DC, int V>
+__global__ __launch_bounds__(kBlock) void sh_fwd_3kn_vec_kernel(
+    int64_t n, int dim, const float* __restrict__ origin, const float* __restrict__ pos,
+    const float* __restrict__ coeffs, const float* __restrict__ dc, const uint32_t* __restrict__ mask,
+    int zero_masked, float* __restrict__ out) {
+    typedef typename VecF<V>::type vf;
+    constexpr int NY = (DEG + 1) * (DEG + 1);
+    const int64_t i = V * ((int64_t)blockIdx.x * kBlock + threadIdx.x);
+    if (i >= n) return;
+    bool ok[V], any = false, all = true;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        ok[j] = mask_ok(mask, i + j);
+        any = any || ok[j];
+        all = all && ok[j];
+    }
+    float r[3 * V];
+#pragma unroll
+    for (int j = 0; j < 3 * V; ++j) r[j] = 0.f;
+    if (any) {
+        float p[3 * V];
+        load3v<V>(pos + 3 * i, p);
+        const f3 o = ld3(origin);
+        f3 dir[V];
+        float Y[V][NY];
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            const f3 diff = mk3(p[3 * j], p[3 * j + 1], p[3 * j + 2]) - o;
+            dir[j] = diff * (1.0f / sqrtf(dot(diff, diff)));
+            sh_basis<DEG>(dir[j], Y[j]);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            vf b[NY];
+#pragma unroll
+            for (int k = 0; k < NY; ++k) {
+                const float* row = HAS_DC ? (k == 0 ? dc + (int64_t)c * n : coeffs + ((int64_t)c * dim + k - 1) * n)
+                                          : coeffs + ((int64_t)c * dim + k) * n;
+                b[k] = __builtin_nontemporal_load(reinterpret_cast<const vf*>(row + i));
+            }
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+                r[3 * j + c] = ok[j] ? sh_color<DEG>(dir[j], Y[j], [&](int k) { return b[k][j]; }) + 0.5f : 0.f;
+        }
+    }
+    if (all || zero_masked) {
+        store3v<V>(out + 3 * i, r);
+    } else {
+#pragma unroll
+        for (int j = 0; j < V; ++j)
+            if (ok[j]) st3(out + 3 * (i + j), mk3(r[3 * j], r[3 * j + 1], r[3 * j + 2]));
+    }
+}
+
+template <int DEG, bool HAS_DC, int V, bool NT>
+__global__ __launch_bounds__(kBlock) void sh_bwd_3kn_vec_kernel(
+    int64_t n, int dim, const float* __restrict__ origin, const float* __restrict__ pos,
+    const float* __restrict__ coeffs, const uint32_t* __restrict__ mask,
+    const float* __restrict__ d_out, float* __restrict__ d_coeffs, float* __restrict__ d_dc,
+    float* __restrict__ d_pos, float* __restrict__ origin_partial) {
+    typedef typename VecF<V>::type vf;
+    constexpr int NY = (DEG + 1) * (DEG + 1);
+    __shared__ float red[3][kBlock / 64];
+    const int64_t i = V * ((int64_t)blockIdx.x * kBlock + threadIdx.x);
+    const bool active = i < n;
+    float go[3 * V], dp[3 * V], Y[V][NY];
+#pragma unroll
+    for (int j = 0; j < 3 * V; ++j) go[j] = dp[j] = 0.f;
+    if (active) {
+        load3v<V>(d_out + 3 * i, go);
+        bool valid[V], need[V], any = false, some = false;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            valid[j] = mask_ok(mask, i + j);
+            if (!valid[j]) go[3 * j] = go[3 * j + 1] = go[3 * j + 2] = 0.f;
+            need[j] = valid[j] && (go[3 * j] != 0.f || go[3 * j + 1] != 0.f || go[3 * j + 2] != 0.f);
+            any = any || need[j];
+            some = some || valid[j];
+#pragma unroll
+            for (int k = 0; k < NY; ++k) Y[j][k] = 0.f;
+        }
+        if (some) {
+            float p[3 * V];
+            load3v<V>(pos + 3 * i, p);
+            const f3 o = ld3(origin);
+            f3 diff[V], dir[V];
+            float il[V];
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                diff[j] = mk3(p[3 * j], p[3 * j + 1], p[3 * j + 2]) - o;
+                il[j] = 1.0f / sqrtf(dot(diff[j], diff[j]));
+                dir[j] = diff[j] * il[j];
+                if (valid[j]) sh_basis<DEG>(dir[j], Y[j]);
+            }
+            if (any) {  // the coefficients enter only the position gradient, times the colour gradient
+                float g[V][NY];
+#pragma unroll
+                for (int k = 0; k < NY; ++k) {
+#pragma unroll
+                    for (int j = 0; j < V; ++j) g[j][k] = 0.f;
+                    if (HAS_DC && k == 0) continue;  // the DC band has no direction dependence
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        const float* row = coeffs + ((int64_t)c * dim + k - (HAS_DC ? 1 : 0)) * n;
+                        const vf b = load_vec<NT>(reinterpret_cast<const vf*>(row + i));
+#pragma unroll
+                        for (int j = 0; j < V; ++j) g[j][k] += b[j] * go[3 * j + c];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    const f3 dd = sh_dir_grad<DEG>(dir[j], g[j]);
+                    // normalize_bwd: (d - (d . n) n) / |v|
+                    const f3 v = dd * il[j] - diff[j] * (il[j] * il[j] * il[j] * dot(dd, diff[j]));
+                    dp[3 * j] = need[j] ? v.x : 0.f;
+                    dp[3 * j + 1] = need[j] ? v.y : 0.f;
+                    dp[3 * j + 2] = need[j] ? v.z : 0.f;
+                }
+            }
+        }
+        store3v<V>(d_pos + 3 * i, dp);
+        // every band of the row, zero above the used degree and for masked Gaussians
+        auto put = [&](float* row, int kk, int c) {
+            vf v;
+#pragma unroll
+            for (int j = 0; j < V; ++j) v[j] = Y[j][kk] * go[3 * j + c];
+            __builtin_nontemporal_store(v, reinterpret_cast<vf*>(row + i));
+        };
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+#pragma unroll
+            for (int k = HAS_DC ? 1 : 0; k < NY; ++k) put(d_coeffs + ((int64_t)c * dim + k - (HAS_DC ? 1 : 0)) * n, k, c);
+            for (int k = NY - (HAS_DC ? 1 : 0); k < dim; ++k)
+                __builtin_nontemporal_store((vf)(0.f), reinterpret_cast<vf*>(d_coeffs + ((int64_t)c * dim + k) * n + i));
+            if (HAS_DC) put(d_dc + (int64_t)c * n, 0, c);
+        }
+    }
+    if (!origin_partial) return;
+    float s[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) s[c] -= dp[3 * j + c];
+    const int t = threadIdx.x, w = t >> 6;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        s[c] = wave_sum(s[c]);
+        if ((t & 63) == 0) red[c][w] = s[c];
+    }
+    __syncthreads();
+    if (t < 3) {
+        float r = 0.f;
+        for (int k = 0; k < kBlock / 64; ++k) r += red[t][k];
+        origin_partial[(int64_t)blockIdx.x * 3 + t] = r;
+    }
+}
+
 // spherical_harmonics_fused_bwd_kernel (sh_bwd.cu:250-315), both layouts. Writes all `dim` bands.
 template <int DEG, bool HAS_DC, bool L3KN>
 __global__ __launch_bounds__(kBlock) void sh_bwd_kernel(
@@ -425,19 +630,45 @@ __global__ __launch_bounds__(kSumThreads) void sum_partials_kernel(const float* 
     }
 }
 
+// Whether every array can be taken V Gaussians at a time (null ones are not used).
+template <int V>
+bool vec_ok(int64_t n, std::initializer_list<const void*> arrays) {
+    uintptr_t bits = 0;
+    for (const void* a : arrays) bits |= (uintptr_t)a;
+    return n % V == 0 && bits % (4 * V) == 0;
+}
+// Gaussians per thread in the [3, K, N] layout: four where a thread's basis values leave room for their rows
+template <int DEG>
+constexpr int kFwdVec = DEG >= 4 ? 2 : 4;
+constexpr int kBwdVec = 2;
+
 template <int DEG, bool DC>
 void launch_fwd(bool l3kn, dim3 g, hipStream_t s, int64_t n, int dim, const float* o, const float* p,
                 const float* c, const float* dc, const uint32_t* m, int zm, float* out) {
-    if (l3kn) sh_fwd_3kn_kernel<DEG, DC><<<g, kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
+    constexpr int V = kFwdVec<DEG>;
+    if (l3kn && 12 * dim * n >= kStreamBytes && vec_ok<V>(n, {p, c, dc, out}))
+        sh_fwd_3kn_vec_kernel<DEG, DC, V><<<xsg_blocks(n / V, kBlock), kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
+    else if (l3kn) sh_fwd_3kn_kernel<DEG, DC><<<g, kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
     else sh_fwd_nk3_kernel<DEG, DC><<<g, kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
 }
 
+// Returns the number of workgroups (origin partials).
 template <int DEG, bool DC>
-void launch_bwd(bool l3kn, dim3 g, hipStream_t s, int64_t n, int dim, const float* o, const float* p,
+unsigned launch_bwd(bool l3kn, dim3 g, hipStream_t s, int64_t n, int dim, const float* o, const float* p,
                 const float* c, const uint32_t* m, const float* dout, float* dcf, float* ddc, float* dp,
                 float* part) {
+    constexpr int V = kBwdVec;
+    if (l3kn && 12 * dim * n >= kVecBytes && vec_ok<V>(n, {p, c, dout, dcf, ddc, dp})) {
+        const unsigned nb = xsg_blocks(n / V, kBlock);
+        if (12 * dim * n >= kStreamBytes)
+            sh_bwd_3kn_vec_kernel<DEG, DC, V, true><<<nb, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
+        else
+            sh_bwd_3kn_vec_kernel<DEG, DC, V, false><<<nb, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
+        return nb;
+    }
     if (l3kn) sh_bwd_kernel<DEG, DC, true><<<g, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
     else sh_bwd_kernel<DEG, DC, false><<<g, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
+    return g.x;
 }
 
 }  // namespace
@@ -508,11 +739,11 @@ int sh_bwd_run(int degree, const float* origin, int64_t n, int dim, const float*
         XSG_TRY_LAUNCH("sh_bwd");
         return XSG_OK;
     }
-    const unsigned nb = xsg_blocks(n, kBlock);
     const bool l = layout_3kn != 0;
-    const dim3 g(nb);
+    const dim3 g(xsg_blocks(n, kBlock));
+    unsigned nb = 0;
 #define XSG_B(D) \
-    (has_dc ? launch_bwd<D, true>(l, g, s, n, dim, origin, positions, coeffs, mask, d_output, d_coeffs, d_coeffs_dc, d_positions, part) \
+    nb = (has_dc ? launch_bwd<D, true>(l, g, s, n, dim, origin, positions, coeffs, mask, d_output, d_coeffs, d_coeffs_dc, d_positions, part) \
             : launch_bwd<D, false>(l, g, s, n, dim, origin, positions, coeffs, mask, d_output, d_coeffs, d_coeffs_dc, d_positions, part))
     switch (degree) {
         case 0: XSG_B(0); break;
