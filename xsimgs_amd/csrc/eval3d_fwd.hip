@@ -14,6 +14,9 @@
 //    after which it changes nothing, so nothing else is selected; a pixel whose transmittance has run out
 //    is a pixel that no alpha reaches (its threshold becomes infinite). Running out is tested once for the
 //    U Gaussians and resolved apart, which each pixel does at most once.
+// The whole op against one pixel per lane, a bit scan per Gaussian and every tile evaluated as M (ro - mu), M rd:
+// 1920x1080, 1 M Gaussians 240 -> 171-190 us; six cameras of 1600x900 886 -> 655; 1237x701 115 -> 85; 2048x128 lidar
+// 72 -> 49; 256x256 63 -> 25; 32 channels at 640x480 170 -> 88; moving origins, which keep that form, 154 -> 154.
 #include <type_traits>
 
 #include "xsg_eval3d.h"
@@ -31,9 +34,8 @@ constexpr int kFwdLdsColors = NT > kTileThreads ? 8 : kFwdColorLdsMax;
 // scalar work of a pair, but a tile is then half as many wavefronts, each twice as long, and its strips share
 // one list: worth it once the grid has many rounds of wavefronts (16 k of two pixels at 1920x1080: 190 us
 // against 194; 68 k for six 1600x900 cameras: 667 against 700; but 6.9 k at 1237x701: 99 against 92), and only
-// where the tile's strips pair up. Where
-// the grid leaves at most four wavefronts per SIMD, the length of a wavefront's chain counts, and U = 4 keeps
-// four evaluations of it in flight (256x256: 24 us against 29).
+// where the tile's strips pair up. Where the grid leaves at most four wavefronts per SIMD, the length of a
+// wavefront's chain counts, and U = 4 keeps four evaluations of it in flight (256x256: 24 us against 29).
 constexpr int64_t kFwdTwoPixelWaves = 8 * 1024;
 constexpr int64_t kFwdDeepWaves = 4 * 1024;
 
