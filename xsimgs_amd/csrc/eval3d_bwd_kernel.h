@@ -707,9 +707,11 @@ int eval3d_bwd_cdim(bool dyn, bool ray_grads, const Eval3dParams& p, hipStream_t
     }
     if constexpr (!wide) {
         if (!ray_grads) {
-            // four pixels per lane when the grid still fills the GPU's wave slots (three waves on each
-            // of 1024 SIMDs); a small grid (a 2048x128 lidar's 1024 tiles) runs two per lane on twice the
-            // waves; the caller may fix either
+            // four pixels per lane when the grid gives each of the 1024 SIMDs three waves of them (three
+            // channels, 100 k Gaussians: 3432 tiles 181 us against 231, 8160 tiles 329 against 411); a small
+            // grid (a 2048x128 lidar's 1024 tiles) runs two per lane on twice the waves (1000 tiles 132
+            // against 155). From 1900 tiles four are ahead by 3 to 8 % there, but with motion or more channels
+            // that was not measured. The caller may fix either
             const bool px4 = p.px_hint == 4 ||
                              (p.px_hint == 0 && (int64_t)n_blocks * (bs4 / 64) >= kBwdFullGridWaves);
             if (tile_px > 128 && px4) {
