@@ -259,6 +259,7 @@ __global__ __launch_bounds__(NT)
     const int32_t range_start = p.offsets[logical];  // utils.h:48-58
     const int32_t range_end = (logical == nblocks - 1) ? (int32_t)g.n_isects : p.offsets[logical + 1];
     const int64_t hw = (int64_t)g.width * g.height;
+    if (past_image(g, trow, tcol)) return;
 
     // strip h's pixel of this lane: its index in the [cams, H, W] images (utils.h:32-44), -1 outside;
     // recomputed where needed rather than kept in registers (opaque: or the compiler keeps it)

@@ -85,6 +85,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     const int32_t range_start = p.offsets[logical];  // utils.h:48-58
     const int32_t range_end = (logical == nblocks - 1) ? (int32_t)g.n_isects : p.offsets[logical + 1];
     const int64_t hw = (int64_t)g.width * g.height;
+    if (past_image(g, trow, tcol)) {
+        if (p.tile_work && tr == 0) p.tile_work[logical] = 0;
+        return;
+    }
 
     // strip h's pixel of this lane: its index in the [cams, H, W] images (utils.h:32-44), -1 outside;
     // recomputed where needed rather than kept in registers (opaque: or the compiler keeps it)
@@ -137,7 +141,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
         for (int k4 = 0; k4 < C4; ++k4) s_col[k4][NT] = make_float4(0.f, 0.f, 0.f, 0.f);
         if constexpr (CL == 0 && CDIM > 0) s_id[NT] = 0;
     }
-    // the tile's first pixel (always inside the image), its middle one and the left end of that one's row
+    // the tile's first pixel, its middle one and the left end of that one's row
     const int64_t p0 = (int64_t)cam * hw + (int64_t)trow * g.tile_h * g.width + tcol * g.tile_w;
     const int64_t ps = p0 + (int64_t)min(g.tile_h / 2, g.height - 1 - trow * g.tile_h) * g.width;
     const f3 o0 = first_origin(ld3(p.ray_o + 3 * p0));

@@ -34,6 +34,12 @@ struct TileGrid {
     int64_t n_isects;
 };
 
+// A tile of a grid larger than the image that has no pixel: its first one, from which a tile's set-up reads
+// rays and times, is past the image (the whole workgroup agrees).
+XSG_DEV bool past_image(const TileGrid& g, int trow, int tcol) {
+    return (int64_t)trow * g.tile_h >= g.height || (int64_t)tcol * g.tile_w >= g.width;
+}
+
 // Rows of M = S^-1 R^T from the raw quaternion (w, x, y, z) and activated scales: row i is column i
 // of R / s_i (utils.h:61-83 and eval3d_fwd.cu:92-107).
 XSG_DEV void iscl_rot_rows(float4 q, f3 s, f3& r0, f3& r1, f3& r2) {
