@@ -1,4 +1,4 @@
-"""The compositor's edge inputs against the float64 oracle: grids larger than the image.
+"""The compositor's edge inputs against the float64 oracle: grids larger than the image, and pixels without a ray.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -145,3 +145,49 @@ def test_grid_larger_than_images_batched():
         for k in ("v_means", "v_quats", "v_scales", "v_opacity", "v_colors"):
             total[k] = total.get(k, 0.0) + one[k]
     _check_grads({k: np_(x) for k, x in zip(("v_means", "v_quats", "v_scales", "v_opacity", "v_colors"), got)}, total)
+
+
+def _spoil(s, where, kind):
+    """Takes the rays of some pixels away: the middle one of every tile, more than a
+    strip of 64, a whole tile."""
+    W, H = s["size"]
+    tw, th = s["tile"]
+    j, i = np.meshgrid(np.arange(W), np.arange(H))
+    if where == "middle":
+        bad = (j % tw == min(tw // 2, W - 1)) & (i % th == min(th // 2, H - 1))
+    elif where == "strip":
+        bad = i % th < min(64 // tw + 1, th // 2)
+    else:
+        bad = (j // tw == 1) & (i // th == 1)
+    if kind == "time":
+        s["rt"] = s["rt"].copy()
+        s["rt"][bad] = np.nan
+    else:
+        s["rd"][bad] = dict(zero=0.0, nan=np.nan)[kind]
+    return bad
+
+
+@pytest.mark.parametrize("tile", [(16, 16), (32, 32), (8, 8)])
+@pytest.mark.parametrize("where", ["middle", "strip", "tile"])
+@pytest.mark.parametrize("kind,moving,dynamic", [("zero", False, False), ("nan", False, False), ("zero", True, False),
+                                                 ("nan", False, True), ("time", False, True), ("zero", False, True)])
+def test_pixels_without_a_ray(kind, moving, dynamic, where, tile):
+    """A zero direction meets every Gaussian at its full opacity, a NaN one at 0.999, and neither changes another
+    pixel. (Their depths are not compared, 0 / 0 in the oracle; gradients are those of the other pixels.)"""
+    W, H = 97, 81
+    s = _scene(W, H, tile, moving=moving, dynamic=dynamic)
+    bad = _spoil(s, where, kind)
+    out, work, T = _forward(s)
+    ref = _oracle_fwd(s)
+    _check_images(out, ref, ~bad)
+    _check_images(out, ref, bad, depth=False)
+    if kind != "zero":
+        return
+    v = _image_grads(W, H, 3)
+    last = np_(out[3]).copy()
+    last[bad] = -1
+    for a in v:
+        a[bad] = 0.0
+    want = _oracle_bwd(s, np_(out[2]), last, v)
+    for kw in (dict(ray_grads=True), dict(ray_grads=False, pixels_per_lane=2), dict(ray_grads=False, pixels_per_lane=4)):
+        _check_grads(_backward(s, out, work, T, v, **kw), want, ~bad)

@@ -289,19 +289,21 @@ __global__ __launch_bounds__(NT)
         const bool inside = pix >= 0;
         const int64_t at = inside ? pix : p0;
         float ik = 0.f;
+        bool ray = true;
         q.x = q.y = 0.f;
         const f3 away = inside ? ld3(p.ray_o + 3 * at) - o0 : mk3(0.f, 0.f, 0.f);
         float rt = 0.f;
         if constexpr (DYN) rt = inside ? p.rtd[at] - rt0 : 0.f;
         if (inside) {
             const f3 ro = ld3(p.ray_o + 3 * at);
-            narrow = narrow && ray_xy(basis, ld3(p.ray_d + 3 * at), q.x, q.y, ik) && finite3(away) && isfinite(rt);
+            ray = ray_xy(basis, ld3(p.ray_d + 3 * at), q.x, q.y, ik) && finite3(away) && isfinite(rt);
+            narrow = narrow && ray;
             same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
                    __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
             far2 = fmaxf(far2, dot(away, away));
             late = fmaxf(late, fabsf(rt));
         }
-        const float4 box = strip_box(inside, q.x, q.y);
+        const float4 box = strip_box(inside, ray, q.x, q.y);
         if (lane == 0) s_box[wave * PX + h] = box;
         const float T_final = 1.0f - p.render_alpha[at];
         q.T = T_final;

@@ -157,21 +157,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
         const int64_t pix = pixel_of(h);
         inside[h] = pix >= 0;
         float ik = 0.f;
+        bool ray = true;
         px[h] = py[h] = 0.f;
         if (inside[h]) {
             const f3 ro = ld3(p.ray_o + 3 * pix), away = ro - o0;
-            narrow = narrow && ray_xy(basis, ld3(p.ray_d + 3 * pix), px[h], py[h], ik);
+            ray = ray_xy(basis, ld3(p.ray_d + 3 * pix), px[h], py[h], ik) && finite3(away);
             same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
                    __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
             far2 = fmaxf(far2, dot(away, away));
-            narrow = narrow && finite3(away);
             if constexpr (DYN) {
                 const float rt = p.rtd ? p.rtd[pix] : 0.f;
-                narrow = narrow && isfinite(rt);
+                ray = ray && isfinite(rt);
                 late = fmaxf(late, fabsf(rt - rt0));
             }
+            narrow = narrow && ray;
         }
-        const float4 box = strip_box(inside[h], px[h], py[h]);
+        const float4 box = strip_box(inside[h], ray, px[h], py[h]);
         if (lane == 0) s_box[wave * PX + h] = box;
         if constexpr (!DYN) s_ik[h][tr] = ik;
     }

@@ -205,14 +205,16 @@ XSG_DEV bool ray_xy(const TileBasis& b, f3 d, float& x, float& y, float& inv_k) 
     return regular_ray(d) && k > 0.0 && k * k > 0.25 * dot64(v, v);
 }
 
-// The box of (x, y) that 64 pixels' rays fill: centre and half extents (hx < 0: no pixel).
-XSG_DEV float4 strip_box(bool inside, float x, float y) {
+// The box of (x, y) that 64 pixels' rays fill: centre and half extents (hx < 0: no pixel; infinite: a pixel
+// whose ray gives no (x, y), or no ray at all, which any Gaussian may reach). Whether there is a pixel is never
+// told from the coordinates, which are NaN then.
+XSG_DEV float4 strip_box(bool inside, bool ray, float x, float y) {
     const float big = __builtin_inff();
     const float x0 = wave_min_f(inside ? x : big), x1 = wave_max_f(inside ? x : -big);
     const float y0 = wave_min_f(inside ? y : big), y1 = wave_max_f(inside ? y : -big);
-    const bool any = x0 <= x1;
-    return make_float4(any ? 0.5f * (x0 + x1) : 0.f, any ? 0.5f * (y0 + y1) : 0.f,
-                       any ? 0.500001f * (x1 - x0) + 1e-7f : -1.f, any ? 0.500001f * (y1 - y0) + 1e-7f : -1.f);
+    if (__ballot(inside) == 0) return make_float4(0.f, 0.f, -1.f, -1.f);
+    if (__ballot(inside && !ray) != 0) return make_float4(0.f, 0.f, big, big);
+    return make_float4(0.5f * (x0 + x1), 0.5f * (y0 + y1), 0.500001f * (x1 - x0) + 1e-7f, 0.500001f * (y1 - y0) + 1e-7f);
 }
 
 // The tile's largest |x| and |y| and its slack (strip_cull), from its strips' and wavefronts'.
