@@ -1,4 +1,5 @@
-"""The compositor's edge inputs against the float64 oracle: grids larger than the image, and pixels without a ray.
+"""The compositor's edge inputs against the float64 oracle: grids larger than the image, pixels without a ray,
+and tiles of very wide rays.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -191,3 +192,51 @@ def test_pixels_without_a_ray(kind, moving, dynamic, where, tile):
     want = _oracle_bwd(s, np_(out[2]), last, v)
     for kw in (dict(ray_grads=True), dict(ray_grads=False, pixels_per_lane=2), dict(ray_grads=False, pixels_per_lane=4)):
         _check_grads(_backward(s, out, work, T, v, **kw), want, ~bad)
+
+
+def _pair_counts(s):
+    """Evaluated pairs of the forward and of the backward (ray gradients, two and four pixels per lane)."""
+    n = [torch.zeros(2, dtype=torch.int64, device="cuda") for _ in range(4)]
+    out, work, T = _forward(s, n[0])
+    v = _image_grads(*s["size"], 3)
+    for c, kw in zip(n[1:], (dict(ray_grads=True), dict(ray_grads=False, pixels_per_lane=2),
+                             dict(ray_grads=False, pixels_per_lane=4))):
+        _backward(s, out, work, T, v, pair_counts=c, **kw)
+    return np.array([int(c[0]) for c in n])
+
+
+@pytest.mark.parametrize("moving,dynamic", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("where", ["middle", "corner"])
+def test_a_pixel_without_a_ray_costs_its_strip(where, moving, dynamic):
+    """One pixel of a 16x16 tile without a ray leaves the tile's other three strips of 64 pixels culled as before."""
+    W, H = 96, 80
+    s = _scene(W, H, (16, 16), moving=moving, dynamic=dynamic)
+    clean = _pair_counts(s)
+    if where == "middle":
+        _spoil(s, "middle", "zero")
+    else:
+        s["rd"][::16, ::16] = 0.0
+    most = clean + (W // 16) * (H // 16) * 64 * s["means"].shape[0]
+    got = _pair_counts(s)
+    print("evaluated", clean, got, "at most", most)
+    assert (got <= most).all()
+
+
+@pytest.mark.parametrize("size,tile,f", [((32, 32), (32, 32), 0.25), ((64, 32), (32, 32), 0.1), ((48, 16), (16, 16), 0.1)])
+def test_wide_tiles(size, tile, f):
+    """Tiles whose corners lie up to 80 degrees from their middle ray are culled too, and stay exact."""
+    W, H = size
+    s = _scene(W, H, tile, f=f)
+    mid = s["rd"][min(tile[1] // 2, H - 1)][tile[0] // 2::tile[0]]
+    angle = max(float(np.degrees(np.arccos((s["rd"][:tile[1], k * tile[0]:(k + 1) * tile[0]] @ m).min())))
+                for k, m in enumerate(mid))
+    assert 62.0 < angle < 84.0, angle
+    out, work, T = _forward(s)
+    _check_images(out, _oracle_fwd(s), np.ones((H, W), bool))
+    v = _image_grads(W, H, 3)
+    ref = _oracle_bwd(s, np_(out[2]), np_(out[3]), v)
+    for kw in (dict(ray_grads=True), dict(ray_grads=False, pixels_per_lane=2), dict(ray_grads=False, pixels_per_lane=4)):
+        _check_grads(_backward(s, out, work, T, v, **kw), ref)
+    n = _pair_counts(s)
+    print("evaluated", n, "of", W * H * s["means"].shape[0], "angle", angle)
+    assert (n <= 0.5 * W * H * s["means"].shape[0]).all()

@@ -263,20 +263,18 @@ __global__ __launch_bounds__(NT)
 
     // strip h's pixel of this lane: its index in the [cams, H, W] images (utils.h:32-44), -1 outside;
     // recomputed where needed rather than kept in registers (opaque: or the compiler keeps it)
-    auto pixel_of = [&](int h) -> int64_t {
-        const int q = (wave * PX + h) * 64 + opaque(lane);
+    auto pixel_at = [&](int q) -> int64_t {
         const int ty = q / g.tile_w, tx = q - ty * g.tile_w;
         const int i = trow * g.tile_h + ty, j = tcol * g.tile_w + tx;
         return q < bs && i < g.height && j < g.width ? (int64_t)cam * hw + (int64_t)i * g.width + j : -1;
     };
+    auto pixel_of = [&](int h) { return pixel_at((wave * PX + h) * 64 + opaque(lane)); };
     // the forward's tile set-up: basis, boxes, whether the rays share one origin
-    const int64_t p0 = (int64_t)cam * hw + (int64_t)trow * g.tile_h * g.width + tcol * g.tile_w;
-    const int64_t ps = p0 + (int64_t)min(g.tile_h / 2, g.height - 1 - trow * g.tile_h) * g.width;
-    const f3 o0 = first_origin(ld3(p.ray_o + 3 * p0));
-    float rt0 = 0.f;
-    if constexpr (DYN) rt0 = first_time(p.rtd[p0]);
-    const TileBasis basis = uniform_basis(
-        tile_basis(ld3(p.ray_d + 3 * (ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w))), ld3(p.ray_d + 3 * ps)));
+    const int64_t ps = (int64_t)cam * hw + (int64_t)min(trow * g.tile_h + g.tile_h / 2, g.height - 1) * g.width + tcol * g.tile_w;
+    const BasisPixel mid = basis_pixel<DYN>(p.ray_o, p.ray_d, p.rtd, ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w), bs, pixel_at);
+    const f3 o0 = mid.o;
+    const float rt0 = mid.t;
+    const TileBasis basis = uniform_basis(tile_basis(mid.d, ld3(p.ray_d + 3 * ps)));
     BwdPixel<CS> px[PX];
     if (tr == 0) put_basis(s_frame, basis);
     bool narrow = true, same = true;
@@ -287,7 +285,7 @@ __global__ __launch_bounds__(NT)
         BwdPixel<CS>& q = px[h];
         const int64_t pix = pixel_of(h);
         const bool inside = pix >= 0;
-        const int64_t at = inside ? pix : p0;
+        const int64_t at = inside ? pix : mid.pix;
         float ik = 0.f;
         bool ray = true;
         q.x = q.y = 0.f;
@@ -300,8 +298,8 @@ __global__ __launch_bounds__(NT)
             narrow = narrow && ray;
             same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
                    __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
-            far2 = fmaxf(far2, dot(away, away));
-            late = fmaxf(late, fabsf(rt));
+            far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
+            late = ray ? fmaxf(late, fabsf(rt)) : late;
         }
         const float4 box = strip_box(inside, ray, q.x, q.y);
         if (lane == 0) s_box[wave * PX + h] = box;
@@ -341,7 +339,7 @@ __global__ __launch_bounds__(NT)
     __syncthreads();
     kind = __builtin_amdgcn_readfirstlane(kind);
     const bool fixed = !DYN && kind == 3;
-    const bool cull = (kind & 1) != 0;
+    const bool rays = (kind & 1) != 0;  // every pixel has one
 
     uint64_t n_eval = 0, n_contrib = 0;  // evaluated / composited pixel-pairs of the wave, when counting
     const int32_t eff_end = min(range_end - 1, __builtin_amdgcn_readfirstlane(tile_max));
@@ -390,7 +388,7 @@ __global__ __launch_bounds__(NT)
                 const float op = p.opac[gid];
                 f3 r0, r1, r2;
                 iscl_rot_rows(q, sc, r0, r1, r2);
-                f3 vel = mk3(0.f, 0.f, 0.f), at = mu;  // at: where the Gaussian is at the first pixel's time
+                f3 vel = mk3(0.f, 0.f, 0.f), at = mu;  // at: where the Gaussian is at the basis pixel's time
                 if constexpr (DYN) {
                     vel = ld3(p.velocity + 3 * gid);
                     at = mu + rt0 * vel;
@@ -415,10 +413,9 @@ __global__ __launch_bounds__(NT)
                     cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy,
                                     s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)),
                                     __builtin_amdgcn_sqrtf(dot(away, away)));
-                    cg.keep_all = cg.keep_all || !cull;
                 }
                 // alphas may reach the clamp, or be no number
-                high = !(op <= kMaxAlpha) || cg.keep_all;
+                high = !(op <= kMaxAlpha) || cg.keep_all || !rays;
                 if constexpr (CL > 0) {
                     const float* cp = p.colors + ((int64_t)fid * CDIM - (int64_t)cam * p.col_shift);
 #pragma unroll

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     __shared__ float4 s_box[NS];                        // the strips' boxes of (x, y)
     __shared__ float s_ik[DYN ? 1 : PX][DYN ? 1 : NT];  // rays of one origin: each pixel's 1 / k
     __shared__ TileFrame s_frame;
-    __shared__ float s_slack[2][NW];  // largest distance from the first pixel's origin, and time from its own
+    __shared__ float s_slack[2][NW];  // largest distance from the basis pixel's origin, and time from its own
     // [wavefront][staging wavefront]: the Gaussians it evaluates, and their number
     __shared__ uint16_t s_list[NW][NW][64 + 2 * U];
     __shared__ int s_cnt[NW][NW];
@@ -92,12 +92,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
 
     // strip h's pixel of this lane: its index in the [cams, H, W] images (utils.h:32-44), -1 outside;
     // recomputed where needed rather than kept in registers (opaque: or the compiler keeps it)
-    auto pixel_of = [&](int h) -> int64_t {
-        const int q = (wave * PX + h) * 64 + opaque(lane);
+    auto pixel_at = [&](int q) -> int64_t {
         const int ty = q / g.tile_w, tx = q - ty * g.tile_w;
         const int i = trow * g.tile_h + ty, j = tcol * g.tile_w + tx;
         return q < bs && i < g.height && j < g.width ? (int64_t)cam * hw + (int64_t)i * g.width + j : -1;
     };
+    auto pixel_of = [&](int h) { return pixel_at((wave * PX + h) * 64 + opaque(lane)); };
     // the conjunction of the wavefronts' votes, written to s_vote before the last barrier
     auto votes = [&]() {
         int v = -1;
@@ -141,14 +141,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
         for (int k4 = 0; k4 < C4; ++k4) s_col[k4][NT] = make_float4(0.f, 0.f, 0.f, 0.f);
         if constexpr (CL == 0 && CDIM > 0) s_id[NT] = 0;
     }
-    // the tile's first pixel, its middle one and the left end of that one's row
-    const int64_t p0 = (int64_t)cam * hw + (int64_t)trow * g.tile_h * g.width + tcol * g.tile_w;
-    const int64_t ps = p0 + (int64_t)min(g.tile_h / 2, g.height - 1 - trow * g.tile_h) * g.width;
-    const f3 o0 = first_origin(ld3(p.ray_o + 3 * p0));
-    float rt0 = 0.f;
-    if constexpr (DYN) rt0 = p.rtd ? first_time(p.rtd[p0]) : 0.f;
-    const TileBasis basis = uniform_basis(
-        tile_basis(ld3(p.ray_d + 3 * (ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w))), ld3(p.ray_d + 3 * ps)));
+    // the left end of the tile's middle row, and the pixel its basis is built on
+    const int64_t ps = (int64_t)cam * hw + (int64_t)min(trow * g.tile_h + g.tile_h / 2, g.height - 1) * g.width + tcol * g.tile_w;
+    const BasisPixel mid = basis_pixel<DYN>(p.ray_o, p.ray_d, p.rtd, ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w), bs, pixel_at);
+    const f3 o0 = mid.o;
+    const float rt0 = mid.t;
+    const TileBasis basis = uniform_basis(tile_basis(mid.d, ld3(p.ray_d + 3 * ps)));
     if (tr == 0) put_basis(s_frame, basis);
     bool narrow = true, same = true;
     float far2 = 0.f, late = 0.f;
@@ -164,12 +162,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
             ray = ray_xy(basis, ld3(p.ray_d + 3 * pix), px[h], py[h], ik) && finite3(away);
             same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
                    __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
-            far2 = fmaxf(far2, dot(away, away));
             if constexpr (DYN) {
-                const float rt = p.rtd ? p.rtd[pix] : 0.f;
+                const float rt = p.rtd ? p.rtd[pix] - rt0 : 0.f;
                 ray = ray && isfinite(rt);
-                late = fmaxf(late, fabsf(rt - rt0));
+                late = ray ? fmaxf(late, fabsf(rt)) : late;
             }
+            far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
             narrow = narrow && ray;
         }
         const float4 box = strip_box(inside[h], ray, px[h], py[h]);
@@ -186,7 +184,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     const int kind = votes();
     // one origin (as float32 values) and ordinary rays: the pairs in the turned frame's affine form
     const bool fixed = !DYN && kind == 3;
-    const bool cull = (kind & 1) != 0;
     if (tr == 0) tile_bounds(s_frame, s_box, nw * PX, s_slack[0], s_slack[1], nw);
     __syncthreads();
 
@@ -232,7 +229,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
                     vel = raw.vel;
                     s_vel[tr] = make_float4(vel.x, vel.y, vel.z, 0.f);
                 }
-                f3 at = mu;  // where the Gaussian is at the first pixel's time
+                f3 at = mu;  // where the Gaussian is at the basis pixel's time
                 if constexpr (DYN) at = mu + rt0 * vel;
                 const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
                 if constexpr (FIXED) {
@@ -249,7 +246,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
                     cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy,
                                     s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)),
                                     __builtin_amdgcn_sqrtf(dot(away, away)));
-                    cg.keep_all = cg.keep_all || !cull;
                 }
                 if constexpr (CL > 0) {
                     const float* cp = p.colors + ((int64_t)fid * CDIM - (int64_t)cam * p.col_shift);

@@ -2,9 +2,10 @@
 //
 // One workgroup per (camera, tile). The tile's pixels form strips of 64 consecutive ones (row-major); a
 // wavefront owns one or more whole strips, one pixel of each per lane. Gaussians of the tile's depth-sorted
-// list are staged in LDS in batches. Tiles whose rays start at one origin (decided by a block vote, always
-// true for a static pinhole, fisheye or spherical camera) work in a turned frame and affine ray coordinates
-// (below); the others with the rows of M = S^-1 R^T, as the reference does per pair.
+// list are staged in LDS in batches. Tiles whose rays all start at one origin, are rays (finite, not zero) and
+// run within 84 degrees of the tile's middle one work in a turned frame and affine ray coordinates (below; a
+// block vote decides, and a static pinhole, fisheye or spherical camera's tiles pass unless they are masked or
+// span half the sphere); the others with the rows of M = S^-1 R^T, as the reference does per pair.
 #pragma once
 #include "xsg_common.h"
 
@@ -103,7 +104,7 @@ XSG_DEV float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfi
 XSG_DEV bool finite3(f3 v) { return isfinite(v.x) && isfinite(v.y) && isfinite(v.z); }
 
 // ---------------------------------------------------------------------------------------------
-// Tiles whose rays share one origin and run within 60 degrees of an axis (every tile of a camera without a
+// Tiles whose rays share one origin and run within 84 degrees of an axis (every tile of a camera without a
 // rolling shutter): two changes of variables make a pair cheap.
 //
 // 1. The frame of a Gaussian is turned until gro = M (o - mu) is (0, 0, D). Everything a pair computes
@@ -113,9 +114,9 @@ XSG_DEV bool finite3(f3 v) { return isfinite(v.x) && isfinite(v.y) && isfinite(v
 //    and the Gaussian's offset from the ray, gro + hit_t grd, is (hit_t t1.d, hit_t t2.d, D tt / |grd|^2).
 //    The turn is the Householder reflection that sends gro to the axis of its largest component (so that
 //    nothing cancels).
-// 2. The tile's rays are d = k (A + x X + y Y) in an orthonormal basis whose A is the tile's middle ray, so
-//    that t1.d / k and the others are affine in the pixel's (x, y): two FMAs each. Power and alpha do not
-//    depend on k; hit_t is 1 / k times what A + x X + y Y gives.
+// 2. The tile's rays are d = k (A + x X + y Y) in an orthonormal basis whose A is the tile's middle ray
+//    (basis_pixel), so that t1.d / k and the others are affine in the pixel's (x, y): two FMAs each. Power and
+//    alpha do not depend on k; hit_t is 1 / k times what A + x X + y Y gives.
 // A pair's alpha then takes 14 FMA-rate instructions instead of 27, its backward 8 fewer again.
 //
 // What float32 would lose is the small difference t.A of a Gaussian near the tile's middle ray, an error of
@@ -190,37 +191,71 @@ XSG_DEV TileBasis get_basis(const TileFrame& f) {
 }
 XSG_DEV f3 uniform3(f3 v) { return mk3(uniform_f(v.x), uniform_f(v.y), uniform_f(v.z)); }
 
-// What a tile's pixels count their origins and times from: the first pixel's, or 0 where that is no number
-// (which must not reach the other pixels).
-XSG_DEV f3 first_origin(f3 o) { return uniform3(finite3(o) ? o : mk3(0.f, 0.f, 0.f)); }
-XSG_DEV float first_time(float t) { return uniform_f(isfinite(t) ? t : 0.f); }
+// The pixel a tile's basis is built on, and whose origin and time its pixels count theirs from: the middle one
+// (pix) or, where that has no ray (a masked pixel), the tile's first one that has. pixel_at(q) is the image index
+// of the tile's q-th pixel, -1 outside; every wavefront looks for itself, with all of its lanes. A tile without
+// any such pixel counts from 0 (what is no number must not reach the other pixels).
+struct BasisPixel {
+    int64_t pix;
+    f3 o, d;
+    float t;
+};
+template <bool DYN, class PixelAt>
+XSG_DEV BasisPixel basis_pixel(const float* ray_o, const float* ray_d, const float* rtd, int64_t pix, int n_pixels,
+                               PixelAt&& pixel_at) {
+    BasisPixel b;
+    auto load = [&](int64_t at) {
+        b.pix = at;
+        b.o = ld3(ray_o + 3 * at);
+        b.d = ld3(ray_d + 3 * at);
+        b.t = 0.f;
+        if constexpr (DYN) b.t = rtd ? rtd[at] : 0.f;
+        return regular_ray(b.d) && finite3(b.o) && isfinite(b.t);
+    };
+    if (!load(pix)) {
+        for (int q = 0; q < n_pixels; q += 64) {
+            const int64_t at = pixel_at(q + (int)__lane_id());
+            const uint64_t m = __ballot(at >= 0 && load(at));
+            if (m == 0) continue;
+            pix = (int64_t)__shfl((long long)at, (int)__builtin_ctzll(m), 64);
+            break;
+        }
+        load(pix);
+    }
+    b.o = uniform3(finite3(b.o) ? b.o : mk3(0.f, 0.f, 0.f));
+    b.t = uniform_f(isfinite(b.t) ? b.t : 0.f);
+    return b;
+}
 
-// A pixel's (x, y) and 1 / k; false where the ray does not run within 60 degrees of the axis.
+// A pixel's (x, y) and 1 / k; false where the ray does not run within 84 degrees of the axis.
 XSG_DEV bool ray_xy(const TileBasis& b, f3 d, float& x, float& y, float& inv_k) {
     const d3 v = to64(d);
     const double k = dot64(v, b.a), r = rcp64(k);
     x = (float)(dot64(v, b.x) * r);
     y = (float)(dot64(v, b.y) * r);
     inv_k = (float)r;
-    return regular_ray(d) && k > 0.0 && k * k > 0.25 * dot64(v, v);
+    return regular_ray(d) && k > 0.0 && k * k > 0.01 * dot64(v, v);
 }
 
 // The box of (x, y) that 64 pixels' rays fill: centre and half extents (hx < 0: no pixel; infinite: a pixel
-// whose ray gives no (x, y), or no ray at all, which any Gaussian may reach). Whether there is a pixel is never
-// told from the coordinates, which are NaN then.
+// whose ray gives no (x, y), or no ray at all, which any Gaussian may reach: that strip alone is then not
+// culled). Whether there is a pixel is never told from the coordinates, which are NaN then.
 XSG_DEV float4 strip_box(bool inside, bool ray, float x, float y) {
     const float big = __builtin_inff();
     const float x0 = wave_min_f(inside ? x : big), x1 = wave_max_f(inside ? x : -big);
     const float y0 = wave_min_f(inside ? y : big), y1 = wave_max_f(inside ? y : -big);
     if (__ballot(inside) == 0) return make_float4(0.f, 0.f, -1.f, -1.f);
     if (__ballot(inside && !ray) != 0) return make_float4(0.f, 0.f, big, big);
-    return make_float4(0.5f * (x0 + x1), 0.5f * (y0 + y1), 0.500001f * (x1 - x0) + 1e-7f, 0.500001f * (y1 - y0) + 1e-7f);
+    return make_float4(0.5f * (x0 + x1), 0.5f * (y0 + y1), 0.500001f * (x1 - x0) + 1.2e-7f * (1.f + fabsf(x0) + fabsf(x1)),
+                       0.500001f * (y1 - y0) + 1.2e-7f * (1.f + fabsf(y0) + fabsf(y1)));
 }
 
-// The tile's largest |x| and |y| and its slack (strip_cull), from its strips' and wavefronts'.
+// The tile's largest |x| and |y| (of the strips that are culled) and its slack (strip_cull), from its strips' and
+// wavefronts'.
 XSG_DEV void tile_bounds(TileFrame& f, const float4* boxes, int n_boxes, const float* far2, const float* late, int nw) {
     float hx = 0.f, hy = 0.f, o = 0.f, t = 0.f;
     for (int k = 0; k < n_boxes; ++k) {
+        if (!(boxes[k].z < __builtin_inff())) continue;
         hx = fmaxf(hx, fabsf(boxes[k].x) + boxes[k].z);
         hy = fmaxf(hy, fabsf(boxes[k].y) + boxes[k].w);
     }
@@ -326,11 +361,11 @@ struct StripCull {
     f3 a1, a2, au;
     float rho2, m1, m2;       // rho^2; margins of t1 and t2
     float xg, yg, ex, ey;     // the ellipse's box
-    bool keep_all, drop_all;
+    bool keep_all;
 };
 
 // hx, hy: the tile's largest |x| and |y|. Where the rays do not share one origin, or the Gaussian moves, the
-// frame belongs to the tile's first pixel, slack bounds how far any pixel's origin or time takes
+// frame belongs to the tile's basis pixel, slack bounds how far any pixel's origin or time takes
 // (o - mu) from there, and d falls short of that frame's by slack / s_min at most; the pairs' float32 error
 // is then about 17 ulp of |gro| (2e-5 of it here). slack < 0: one origin.
 XSG_DEV StripCull strip_cull(const RayFrame& f, f3 mu, f3 s, float4 q, float op, float hx, float hy, float slack,
@@ -351,8 +386,8 @@ XSG_DEV StripCull strip_cull(const RayFrame& f, f3 mu, f3 s, float4 q, float op,
         sane = s_min * s_min * 1e12f >= dist + slack;  // the pairs' products stay finite
     }
     const float room = f.D * f.D - lim * lim;
-    c.drop_all = ok && op < 1.f / 255.f;
-    c.keep_all = !ok || !sane || !(room > 1e-3f * lim * lim);
+    const bool drop_all = ok && op < 1.f / 255.f;
+    c.keep_all = !drop_all && (!ok || !sane || !(room > 1e-3f * lim * lim));
     c.rho2 = lim * lim * __builtin_amdgcn_rcpf(room) * 1.0001f;
     const float u_max = fabsf(f.au.x) + fabsf(f.au.y) * hx + fabsf(f.au.z) * hy;
     c.m1 = 1e-6f * (fabsf(f.a1.x) + fabsf(f.a1.y) * hx + fabsf(f.a1.z) * hy);
@@ -369,10 +404,12 @@ XSG_DEV StripCull strip_cull(const RayFrame& f, f3 mu, f3 s, float4 q, float op,
                   det_err * fabsf(c.xg)) * 1.0002f;
     c.ey = aid * (reach * __builtin_amdgcn_sqrtf(f.a1.y * f.a1.y + f.a2.y * f.a2.y) + 4e-6f * (fabsf(ny0) + fabsf(ny1)) +
                   det_err * fabsf(c.yg)) * 1.0002f;
+    c.ex = drop_all ? -__builtin_inff() : c.ex;  // out of every finite box
     return c;
 }
 
-// True unless no pixel of the strip can take the Gaussian (every comparison fails on a NaN).
+// True unless no pixel of the strip can take the Gaussian (every comparison fails on a NaN, so none of them
+// drops a Gaussian from an infinite box).
 XSG_DEV bool strip_keep(float4 box, const StripCull& c) {
     const float b1 = fabsf(fmaf(box.y, c.a1.z, fmaf(box.x, c.a1.y, c.a1.x))) - fabsf(c.a1.y) * box.z - fabsf(c.a1.z) * box.w;
     const float b2 = fabsf(fmaf(box.y, c.a2.z, fmaf(box.x, c.a2.y, c.a2.x))) - fabsf(c.a2.y) * box.z - fabsf(c.a2.z) * box.w;
@@ -380,7 +417,7 @@ XSG_DEV bool strip_keep(float4 box, const StripCull& c) {
     const float n1 = fmaxf(0.f, b1 - c.m1), n2 = fmaxf(0.f, b2 - c.m2);
     const bool out = n1 * n1 + n2 * n2 > c.rho2 * bu * bu || fabsf(box.x - c.xg) > box.z + c.ex ||
                      fabsf(box.y - c.yg) > box.w + c.ey;
-    return box.z >= 0.f && !c.drop_all && (c.keep_all || !out);
+    return box.z >= 0.f && (c.keep_all || !out);
 }
 
 // Lane-to-lane moves inside rows of 16 lanes (DPP). `update_dpp` with all rows/banks enabled and
