@@ -1,5 +1,5 @@
 """The compositor's edge inputs against the float64 oracle: grids larger than the image, pixels without a ray,
-and tiles of very wide rays.
+tiles of very wide rays, and flat Gaussians seen from moving origins.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -240,3 +240,29 @@ def test_wide_tiles(size, tile, f):
     n = _pair_counts(s)
     print("evaluated", n, "of", W * H * s["means"].shape[0], "angle", angle)
     assert (n <= 0.5 * W * H * s["means"].shape[0]).all()
+
+
+@pytest.mark.parametrize("dynamic", [False, True])
+@pytest.mark.parametrize("flat", [1.0, 1e-2, 1e-3])
+@pytest.mark.parametrize("tile", [(16, 16), (32, 32)])
+def test_flat_gaussians_from_moving_origins(tile, flat, dynamic):
+    """Origins that move by many times a flat Gaussian's thickness within a tile leave it culled by its other axes,
+    and no pair is lost. Bound on the pairs: twice those of one origin, the ball that the motion adds to every
+    Gaussian being smaller than its larger axes. The last ids and images are the oracle's but for the pairs that
+    float32 cannot decide: its alpha is off by 17 ulp of |o - mu| / s_min there."""
+    W, H = 96, 80
+    s = _scene(W, H, tile, moving=True, dynamic=dynamic, n=300, seed=5)
+    s["scales"][:, 0] = s["scales"].max(1) * flat
+    still = dict(s, ro=np.ascontiguousarray(np.broadcast_to(s["ro"][H // 2, W // 2], s["ro"].shape)))
+    if dynamic:
+        still["rt"] = np.zeros_like(s["rt"])
+    most = 2 * _pair_counts(still)
+    n = _pair_counts(s)
+    print("evaluated", n, "one origin", most // 2)
+    assert (n <= most).all()
+    out, work, T = _forward(s)
+    ref = _oracle_fwd(s)
+    share = 1e-4 if flat == 1.0 else 1e-2
+    for got, want in zip((out[0], out[2]), (ref[0], ref[2])):
+        assert (np.abs(np_(got) - want) > 1e-3).mean() <= share
+    assert (np_(out[3]) != ref[3]).mean() <= share

@@ -386,6 +386,7 @@ __global__ __launch_bounds__(NT)
                 const float4 q = p.quats[gid];
                 const f3 sc = ld3(p.scales + 3 * gid);
                 const float op = p.opac[gid];
+                const CullInput in = cull_input(mu, sc, q, op);
                 f3 r0, r1, r2;
                 iscl_rot_rows(q, sc, r0, r1, r2);
                 f3 vel = mk3(0.f, 0.f, 0.f), at = mu;  // at: where the Gaussian is at the basis pixel's time
@@ -393,14 +394,13 @@ __global__ __launch_bounds__(NT)
                     vel = ld3(p.velocity + 3 * gid);
                     at = mu + rt0 * vel;
                 }
-                const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
                 if constexpr (FIXED) {
+                    const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
                     slot[0] = make_float4(f.a1.x, f.a1.y, f.a1.z, f.D * f.D * -0.72134752f);
                     slot[1] = make_float4(f.a2.x, f.a2.y, f.a2.z, f.D);
                     slot[2] = make_float4(f.au.x, f.au.y, f.au.z, op);
-                    cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy, -1.f, 0.f);
+                    cg = strip_cull(f, in, s_frame.hx, s_frame.hy);
                 } else {
-                    const f3 away = at - o0;
                     slot[0] = make_float4(r0.x, r0.y, r0.z, mu.x);
                     slot[1] = make_float4(r1.x, r1.y, r1.z, mu.y);
                     slot[2] = make_float4(r2.x, r2.y, r2.z, mu.z);
@@ -410,9 +410,8 @@ __global__ __launch_bounds__(NT)
                         s_vel[tr] = make_float4(vel.x, vel.y, vel.z, 0.f);
                         s_mv[tr] = make_float4(mv.x, mv.y, mv.z, 0.f);
                     }
-                    cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy,
-                                    s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)),
-                                    __builtin_amdgcn_sqrtf(dot(away, away)));
+                    cg = strip_cull_moving(r0, r1, r2, at, sc, in, o0,
+                                           s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)), s_frame);
                 }
                 // alphas may reach the clamp, or be no number
                 high = !(op <= kMaxAlpha) || cg.keep_all || !rays;

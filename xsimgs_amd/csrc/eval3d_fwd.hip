@@ -222,6 +222,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
                 const f3 mu = raw.mu, sc = raw.sc;
                 const float4 q = raw.q;
                 const float op = raw.op;
+                const CullInput in = cull_input(mu, sc, q, op);
                 f3 r0, r1, r2;
                 iscl_rot_rows(q, sc, r0, r1, r2);
                 f3 vel = mk3(0.f, 0.f, 0.f);
@@ -231,21 +232,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
                 }
                 f3 at = mu;  // where the Gaussian is at the basis pixel's time
                 if constexpr (DYN) at = mu + rt0 * vel;
-                const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
                 if constexpr (FIXED) {
+                    const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
                     s_m0[tr] = make_float4(f.a1.x, f.a1.y, f.a1.z, f.D * f.D * -0.72134752f);
                     s_m1[tr] = make_float4(f.a2.x, f.a2.y, f.a2.z, f.D);
                     s_m2[tr] = make_float4(f.au.x, f.au.y, f.au.z, op);
-                    cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy, -1.f, 0.f);
+                    cg = strip_cull(f, in, s_frame.hx, s_frame.hy);
                 } else {
-                    const f3 away = at - o0;
                     s_m0[tr] = make_float4(r0.x, r0.y, r0.z, mu.x);
                     s_m1[tr] = make_float4(r1.x, r1.y, r1.z, mu.y);
                     s_m2[tr] = make_float4(r2.x, r2.y, r2.z, mu.z);
                     if constexpr (!OP_IN_COL) s_op[tr].x = op;
-                    cg = strip_cull(f, mu, sc, q, op, s_frame.hx, s_frame.hy,
-                                    s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)),
-                                    __builtin_amdgcn_sqrtf(dot(away, away)));
+                    cg = strip_cull_moving(r0, r1, r2, at, sc, in, o0,
+                                           s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)), s_frame);
                 }
                 if constexpr (CL > 0) {
                     const float* cp = p.colors + ((int64_t)fid * CDIM - (int64_t)cam * p.col_shift);

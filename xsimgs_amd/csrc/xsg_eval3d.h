@@ -364,30 +364,38 @@ struct StripCull {
     bool keep_all;
 };
 
-// hx, hy: the tile's largest |x| and |y|. Where the rays do not share one origin, or the Gaussian moves, the
-// frame belongs to the tile's basis pixel, slack bounds how far any pixel's origin or time takes
-// (o - mu) from there, and d falls short of that frame's by slack / s_min at most; the pairs' float32 error
-// is then about 17 ulp of |gro| (2e-5 of it here). slack < 0: one origin.
-XSG_DEV StripCull strip_cull(const RayFrame& f, f3 mu, f3 s, float4 q, float op, float hx, float hy, float slack,
-                             float dist) {
-    StripCull c;
-    c.a1 = f.a1; c.a2 = f.a2; c.au = f.au;
+// d_lim: sqrt(2 ln(255 op)) through log2; + 3e-3 covers the rounding of log, exp, the product and the compare.
+XSG_DEV float reach_of(float op) {
+    const float l2 = 2.f * 0.69314718f * __builtin_amdgcn_logf(fmaxf(255.f * op, 1.f));
+    return __builtin_amdgcn_sqrtf(l2) * 1.0001f + 3e-3f;
+}
+
+// What of a Gaussian the test needs beside its frame, taken before it (its inputs then end there).
+struct CullInput {
+    float lim;       // d_lim
+    bool ok, low;    // finite and not degenerate; below the alpha threshold everywhere
+};
+XSG_DEV CullInput cull_input(f3 mu, f3 s, float4 q, float op) {
     const float s_max = fmaxf(s.x, fmaxf(s.y, s.z)), s_min = fminf(s.x, fminf(s.y, s.z));
     const float q2 = q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w;
-    const bool ok = finite3(mu) && s_min >= 1e-12f && s_max <= 1e9f && q2 >= 1e-30f && q2 <= 1e30f && isfinite(op) &&
-                    fabsf(f.D) < 1e15f;
+    CullInput c;
+    c.ok = finite3(mu) && s_min >= 1e-12f && s_max <= 1e9f && q2 >= 1e-30f && q2 <= 1e30f && isfinite(op);
+    c.low = op < 1.f / 255.f;
     // 2 ln(255 op) through log2; + 3e-3 covers the rounding of log, exp, the product and the compare
     const float l2 = 2.f * 0.69314718f * __builtin_amdgcn_logf(fmaxf(255.f * op, 1.f));
-    float lim = __builtin_amdgcn_sqrtf(l2) * 1.0001f + 3e-3f;
-    bool sane = true;
-    if (slack >= 0.f) {
-        const float inv_smin = __builtin_amdgcn_rcpf(s_min) * 1.00001f;
-        lim += inv_smin * (slack * 1.00001f + 2e-5f * (dist + slack));
-        sane = s_min * s_min * 1e12f >= dist + slack;  // the pairs' products stay finite
-    }
+    c.lim = __builtin_amdgcn_sqrtf(l2) * 1.0001f + 3e-3f;
+    return c;
+}
+
+// hx, hy: the tile's largest |x| and |y|.
+XSG_DEV StripCull strip_cull(const RayFrame& f, const CullInput& in, float hx, float hy) {
+    StripCull c;
+    c.a1 = f.a1; c.a2 = f.a2; c.au = f.au;
+    const float lim = in.lim;
+    const bool ok = in.ok && fabsf(f.D) < 1e15f;
     const float room = f.D * f.D - lim * lim;
-    const bool drop_all = ok && op < 1.f / 255.f;
-    c.keep_all = !drop_all && (!ok || !sane || !(room > 1e-3f * lim * lim));
+    const bool drop_all = ok && in.low;
+    c.keep_all = !drop_all && (!ok || !(room > 1e-3f * lim * lim));
     c.rho2 = lim * lim * __builtin_amdgcn_rcpf(room) * 1.0001f;
     const float u_max = fabsf(f.au.x) + fabsf(f.au.y) * hx + fabsf(f.au.z) * hy;
     c.m1 = 1e-6f * (fabsf(f.a1.x) + fabsf(f.a1.y) * hx + fabsf(f.a1.z) * hy);
@@ -406,6 +414,27 @@ XSG_DEV StripCull strip_cull(const RayFrame& f, f3 mu, f3 s, float4 q, float op,
                   det_err * fabsf(c.yg)) * 1.0002f;
     c.ex = drop_all ? -__builtin_inff() : c.ex;  // out of every finite box
     return c;
+}
+
+// The same where the rays do not share one origin, or the Gaussian moves. The frame belongs to the tile's basis
+// pixel (origin o0, the Gaussian then at `at`), and slack bounds how far any pixel's origin or time takes
+// (o - mu) from there: the ellipsoid of semi-axes d_lim s_i that such a ray must meet, widened by a ball of that
+// radius, lies in the one of semi-axes sqrt((1 + 1 / p) (d_lim s_i)^2 + (1 + p) slack^2) for every p > 0. p is
+// d_lim s_min / slack, for which the thinnest axis grows by slack alone, but at least 3: the axes of a flat Gaussian
+// then grow by 15 %, or to twice the slack. (Widening by slack / s_min instead, which is exact for a ball, kept
+// nearly everything of a flat one.) The pairs' float32 error, about 17 ulp of |gro|, adds to d_lim (2e-5 of it here).
+XSG_DEV StripCull strip_cull_moving(f3 r0, f3 r1, f3 r2, f3 at, f3 s, CullInput in, f3 o0, float slack,
+                                    const TileFrame& tile) {
+    const f3 away = at - o0;
+    const float far = __builtin_amdgcn_sqrtf(dot(away, away)) + slack, s_min = fminf(s.x, fminf(s.y, s.z));
+    in.ok = in.ok && s_min * s_min * 1e12f >= far;  // the pairs' products stay finite
+    in.lim += 2.00001e-5f * far * __builtin_amdgcn_rcpf(s_min);
+    const float ball = fmaxf(slack * 1.00001f, 1e-20f);
+    const float p = fmaxf(3.f, in.lim * s_min * __builtin_amdgcn_rcpf(ball)), a = 1.f + __builtin_amdgcn_rcpf(p);
+    const float w = ball * __builtin_amdgcn_rcpf(in.lim), b = (1.f + p) * w * w;
+    const RayFrame f = ray_frame(s.x * __builtin_amdgcn_rsqf(a * s.x * s.x + b) * r0, s.y * __builtin_amdgcn_rsqf(a * s.y * s.y + b) * r1,
+                                 s.z * __builtin_amdgcn_rsqf(a * s.z * s.z + b) * r2, at, o0, get_basis(tile));
+    return strip_cull(f, in, tile.hx, tile.hy);
 }
 
 // True unless no pixel of the strip can take the Gaussian (every comparison fails on a NaN, so none of them
