@@ -269,13 +269,42 @@ __global__ __launch_bounds__(NT)
         return q < bs && i < g.height && j < g.width ? (int64_t)cam * hw + (int64_t)i * g.width + j : -1;
     };
     auto pixel_of = [&](int h) { return pixel_at((wave * PX + h) * 64 + opaque(lane)); };
-    // the forward's tile set-up: basis, boxes, whether the rays share one origin
+    // The left end of the tile's middle row, and that row's middle pixel (which stands in for those outside)
     const int64_t ps = (int64_t)cam * hw + (int64_t)min(trow * g.tile_h + g.tile_h / 2, g.height - 1) * g.width + tcol * g.tile_w;
-    const BasisPixel mid = basis_pixel<DYN>(p.ray_o, p.ray_d, p.rtd, ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w), bs, pixel_at);
+    const int64_t pm = ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w);
+    // The pixels' state and rays, loaded before the basis pixel's is looked at (their latencies overlap)
+    BwdPixel<CS> px[PX];
+    f3 ray_o[PX], ray_d[PX];
+    float ray_t[PX];
+    bool inside[PX];
+#pragma unroll
+    for (int h = 0; h < PX; ++h) {
+        BwdPixel<CS>& q = px[h];
+        const int64_t pix = pixel_of(h);
+        inside[h] = pix >= 0;
+        const int64_t at = inside[h] ? pix : pm;
+        ray_o[h] = ld3(p.ray_o + 3 * at);
+        ray_d[h] = ld3(p.ray_d + 3 * at);
+        ray_t[h] = 0.f;
+        if constexpr (DYN) ray_t[h] = p.rtd[at];
+        const float T_final = 1.0f - p.render_alpha[at];
+        q.T = T_final;
+#pragma unroll
+        for (int k = 0; k < CS; ++k) q.v_c[k] = 0.f;
+#pragma unroll
+        for (int k = 0; k < CDIM; ++k) q.v_c[k] = inside[h] ? p.v_rgb[at * CDIM + k] : 0.0f;
+        q.v_d = inside[h] ? p.v_depth[at] : 0.0f;
+        q.buf = inside[h] ? -T_final * p.v_alpha[at] : 0.0f;
+        q.bin_final = inside[h] ? p.last_ids[at] : -1;
+        q.v_ro = mk3(0.f, 0.f, 0.f);
+        q.v_rd = mk3(0.f, 0.f, 0.f);
+    }
+    // the forward's tile set-up: basis, boxes, whether the rays share one origin
+    const f3 side = ld3(p.ray_d + 3 * ps);
+    const BasisPixel mid = basis_pixel<DYN>(p.ray_o, p.ray_d, p.rtd, pm, bs, pixel_at);
     const f3 o0 = mid.o;
     const float rt0 = mid.t;
-    const TileBasis basis = uniform_basis(tile_basis(mid.d, ld3(p.ray_d + 3 * ps)));
-    BwdPixel<CS> px[PX];
+    const TileBasis basis = uniform_basis(tile_basis(mid.d, side));
     if (tr == 0) put_basis(s_frame, basis);
     bool narrow = true, same = true;
     float far2 = 0.f, late = 0.f;
@@ -283,41 +312,25 @@ __global__ __launch_bounds__(NT)
 #pragma unroll
     for (int h = 0; h < PX; ++h) {
         BwdPixel<CS>& q = px[h];
-        const int64_t pix = pixel_of(h);
-        const bool inside = pix >= 0;
-        const int64_t at = inside ? pix : mid.pix;
         float ik = 0.f;
         bool ray = true;
         q.x = q.y = 0.f;
-        const f3 away = inside ? ld3(p.ray_o + 3 * at) - o0 : mk3(0.f, 0.f, 0.f);
-        float rt = 0.f;
-        if constexpr (DYN) rt = inside ? p.rtd[at] - rt0 : 0.f;
-        if (inside) {
-            const f3 ro = ld3(p.ray_o + 3 * at);
-            ray = ray_xy(basis, ld3(p.ray_d + 3 * at), q.x, q.y, ik) && finite3(away) && isfinite(rt);
+        if (inside[h]) {
+            const f3 ro = ray_o[h], away = ro - o0;
+            const float rt = ray_t[h] - rt0;
+            ray = ray_xy(basis, ray_d[h], q.x, q.y, ik) && finite3(away) && isfinite(rt);
             narrow = narrow && ray;
             same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
                    __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
             far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
             late = ray ? fmaxf(late, fabsf(rt)) : late;
         }
-        const float4 box = strip_box(inside, ray, q.x, q.y);
+        const float4 box = strip_box(inside[h], ray, q.x, q.y);
         if (lane == 0) s_box[wave * PX + h] = box;
-        const float T_final = 1.0f - p.render_alpha[at];
-        q.T = T_final;
-#pragma unroll
-        for (int k = 0; k < CS; ++k) q.v_c[k] = 0.f;
-#pragma unroll
-        for (int k = 0; k < CDIM; ++k) q.v_c[k] = inside ? p.v_rgb[at * CDIM + k] : 0.0f;
-        q.v_d = inside ? p.v_depth[at] : 0.0f;
         q.v_t = ik;  // until the mode is known
-        q.buf = inside ? -T_final * p.v_alpha[at] : 0.0f;
-        q.bin_final = inside ? p.last_ids[at] : -1;
         const int m = wave_max(q.bin_final);
         if (lane == 0) s_sbf[wave * PX + h] = m;
         wave_bin_final = max(wave_bin_final, m);
-        q.v_ro = mk3(0.f, 0.f, 0.f);
-        q.v_rd = mk3(0.f, 0.f, 0.f);
     }
     {
         const int v = (__ballot(!narrow) == 0 ? 1 : 0) | (__ballot(!same) == 0 ? 2 : 0);

@@ -141,33 +141,41 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
         for (int k4 = 0; k4 < C4; ++k4) s_col[k4][NT] = make_float4(0.f, 0.f, 0.f, 0.f);
         if constexpr (CL == 0 && CDIM > 0) s_id[NT] = 0;
     }
+    // The pixels' rays and times, loaded before the basis pixel's is looked at (their latencies overlap)
+    f3 ray_o[PX], ray_d[PX];
+    float ray_t[PX];
+#pragma unroll
+    for (int h = 0; h < PX; ++h) {
+        const int64_t pix = pixel_of(h);
+        inside[h] = pix >= 0;
+        ray_o[h] = inside[h] ? ld3(p.ray_o + 3 * pix) : mk3(0.f, 0.f, 0.f);
+        ray_d[h] = inside[h] ? ld3(p.ray_d + 3 * pix) : mk3(0.f, 0.f, 0.f);
+        ray_t[h] = 0.f;
+        if constexpr (DYN) ray_t[h] = inside[h] && p.rtd ? p.rtd[pix] : 0.f;
+    }
     // the left end of the tile's middle row, and the pixel its basis is built on
     const int64_t ps = (int64_t)cam * hw + (int64_t)min(trow * g.tile_h + g.tile_h / 2, g.height - 1) * g.width + tcol * g.tile_w;
+    const f3 side = ld3(p.ray_d + 3 * ps);
     const BasisPixel mid = basis_pixel<DYN>(p.ray_o, p.ray_d, p.rtd, ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w), bs, pixel_at);
     const f3 o0 = mid.o;
     const float rt0 = mid.t;
-    const TileBasis basis = uniform_basis(tile_basis(mid.d, ld3(p.ray_d + 3 * ps)));
+    const TileBasis basis = uniform_basis(tile_basis(mid.d, side));
     if (tr == 0) put_basis(s_frame, basis);
     bool narrow = true, same = true;
     float far2 = 0.f, late = 0.f;
 #pragma unroll
     for (int h = 0; h < PX; ++h) {
-        const int64_t pix = pixel_of(h);
-        inside[h] = pix >= 0;
         float ik = 0.f;
         bool ray = true;
         px[h] = py[h] = 0.f;
         if (inside[h]) {
-            const f3 ro = ld3(p.ray_o + 3 * pix), away = ro - o0;
-            ray = ray_xy(basis, ld3(p.ray_d + 3 * pix), px[h], py[h], ik) && finite3(away);
+            const f3 ro = ray_o[h], away = ro - o0;
+            const float rt = ray_t[h] - rt0;
+            ray = ray_xy(basis, ray_d[h], px[h], py[h], ik) && finite3(away) && isfinite(rt);
             same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
                    __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
-            if constexpr (DYN) {
-                const float rt = p.rtd ? p.rtd[pix] - rt0 : 0.f;
-                ray = ray && isfinite(rt);
-                late = ray ? fmaxf(late, fabsf(rt)) : late;
-            }
             far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
+            late = ray ? fmaxf(late, fabsf(rt)) : late;
             narrow = narrow && ray;
         }
         const float4 box = strip_box(inside[h], ray, px[h], py[h]);
