@@ -1,5 +1,5 @@
 """The compositor's edge inputs against the float64 oracle: grids larger than the image, pixels without a ray,
-tiles of very wide rays, and flat Gaussians seen from moving origins.
+tiles of very wide rays, flat Gaussians seen from moving origins, and Gaussians whose turn is a near tie.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -266,3 +266,46 @@ def test_flat_gaussians_from_moving_origins(tile, flat, dynamic):
     for got, want in zip((out[0], out[2]), (ref[0], ref[2])):
         assert (np.abs(np_(got) - want) > 1e-3).mean() <= share
     assert (np_(out[3]) != ref[3]).mean() <= share
+
+
+def _quat_mul(a, b):
+    w1, x1, y1, z1 = a.T
+    w2, x2, y2, z2 = b.T
+    return np.stack([w1 * w2 - x1 * x2 - y1 * y2 - z1 * z2, w1 * x2 + x1 * w2 + y1 * z2 - z1 * y2,
+                     w1 * y2 - x1 * z2 + y1 * w2 + z1 * x2, w1 * z2 + x1 * y2 - y1 * x2 + z1 * w2], 1)
+
+
+def test_turn_of_near_ties():
+    """The largest components of M (o - mu) agree to about an ulp, so that rounding picks the axis of the turn: the
+    backward turns the gradients back about the axis that it turned them by. Per Gaussian: 1e-3 of the gradient,
+    the suite's bar, for those of at least a fifth of the usual size."""
+    W = H = 64
+    per, tile = 400, (16, 16)
+    g = np.random.default_rng(2)
+    s = _scene(W, H, tile, n=1, f=0.8)
+    n = per * s["offsets"].size
+    t = np.repeat(np.arange(s["offsets"].size), per)
+    v = -s["rd"][t // 4 * 16 + g.integers(0, 16, n), t % 4 * 16 + g.integers(0, 16, n)].astype(np.float64)
+    z = np.sort(g.uniform(3, 12, (s["offsets"].size, per)), 1).reshape(-1, 1)
+    scales = np.exp(g.normal(-2.0, 0.4, (n, 3)))
+    gro = np.where(np.arange(3) == g.integers(0, 4, n)[:, None], g.uniform(0.1, 0.95, (n, 1)), 1.0)
+    a = gro * g.choice([-1.0, 1.0], (n, 3)) * scales  # R^T (o - mu), up to its length
+    a /= np.linalg.norm(a, axis=1, keepdims=True)
+    arc = np.concatenate([1 + (a * v).sum(1, keepdims=True), np.cross(a, v)], 1)  # the rotation that takes a to v
+    arc /= np.linalg.norm(arc, axis=1, keepdims=True)
+    half = g.uniform(0, np.pi, (n, 1))
+    quats = _quat_mul(np.concatenate([np.cos(half), np.sin(half) * v], 1), arc)
+    f32 = lambda x: np.ascontiguousarray(x, np.float32)
+    s.update(means=f32(s["ro"][0, 0] - v * z), quats=f32(quats), scales=f32(scales), colors=f32(g.normal(0, 1, (n, 3))),
+             opac=f32(g.uniform(0.006, 0.02, n)), flat=np.arange(n, dtype=np.int32),
+             offsets=(np.arange(s["offsets"].size, dtype=np.int32) * per).reshape(s["offsets"].shape))
+    out, work, T = _forward(s)
+    grads = _image_grads(W, H, 3)
+    ref = _oracle_bwd(s, np_(out[2]), np_(out[3]), grads)
+    for kw in (dict(ray_grads=True), dict(ray_grads=False, pixels_per_lane=2), dict(ray_grads=False, pixels_per_lane=4)):
+        got = _backward(s, out, work, T, grads, **kw)
+        for name in ("v_means", "v_quats", "v_scales"):
+            size = np.linalg.norm(ref[name], axis=1)
+            usual = size > np.quantile(size, 0.2)
+            err = np.linalg.norm(got[name] - ref[name], axis=1)
+            assert (err[usual] <= 1e-3 * size[usual]).all(), (name, int((err[usual] > 1e-3 * size[usual]).sum()), kw)

@@ -267,10 +267,17 @@ XSG_DEV void tile_bounds(TileFrame& f, const float4* boxes, int n_boxes, const f
 }
 
 // One Gaussian's turned frame (rows in world space) and its affine rows (value, d/dx, d/dy).
+// The turn: which component of gro is the largest (x, else y, else z) and whether it is negative. Whoever turns
+// back takes it from here: another copy of the code may round a near tie the other way, and turn about another
+// axis.
+struct Turn {
+    bool kx, ky, neg;
+};
 struct RayFrame {
     f3 t1, t2, u;
     f3 a1, a2, au;
     float D;
+    Turn turn;
 };
 
 XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& bas) {
@@ -287,6 +294,7 @@ XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& ba
     const float beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;  // at the Gaussian's centre any frame will do
     const f3 w = ga * ra + gb * rb + vk * rk;
     RayFrame f;
+    f.turn = Turn{kx, ky, signbit(gk)};
     f.t1 = ra - (beta * ga) * w;
     f.t2 = rb - (beta * gb) * w;
     f.u = copysignf(1.0f, gk) * ((beta * vk) * w - rk);
@@ -303,17 +311,16 @@ XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& ba
 }
 
 // A vector and a symmetric matrix (upper triangle, row-major) of the turned frame, turned back into the
-// Gaussian's own normalised frame; the rows, mean and origin are those ray_frame was given.
-XSG_DEV void turn_back(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, f3& v, float (&Q)[6]) {
+// Gaussian's own normalised frame; the rows, mean and origin are those ray_frame was given, the turn its own.
+XSG_DEV void turn_back(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, Turn turn, f3& v, float (&Q)[6]) {
     const f3 g = rows_mul(r0, r1, r2, o - mu);
-    const float ax = fabsf(g.x), ay = fabsf(g.y), az = fabsf(g.z);
-    const bool kx = ax >= ay && ax >= az, ky = !kx && ay >= az;
+    const bool kx = turn.kx, ky = turn.ky;
     const float gk = kx ? g.x : ky ? g.y : g.z, ga = kx ? g.y : g.x, gb = (kx || ky) ? g.z : g.y;
     const float D = __builtin_amdgcn_sqrtf(dot(g, g));
-    const float vk = gk + copysignf(D, gk);
+    const float vk = gk + (turn.neg ? -D : D);
     const float den = D * (D + fabsf(gk));
     const float beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;
-    const float s = -copysignf(1.0f, gk);  // u is s times the reflected row k
+    const float s = turn.neg ? 1.0f : -1.0f;  // u is s times the reflected row k
     const f3 n = mk3(ga, gb, vk);
     f3 w = mk3(v.x, v.y, s * v.z);
     w = w - (beta * dot(n, w)) * n;  // in the order (a, b, k)
