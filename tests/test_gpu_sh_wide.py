@@ -1,9 +1,10 @@
 """The [3, K, N] colour kernels that take several Gaussians per thread, against the one-per-thread kernels.
 
-The wide kernels run on large arrays whose length is a multiple of their vector; one Gaussian more (an odd
-length) takes the kernels that the other tests hold against the oracle, on the same values. Sizes: just above
-the backward's rule (48 MB of coefficients) with a last workgroup partly filled and lengths of 2 modulo 4, and
-just above the forward's (192 MB).
+The wide kernels run from degree 3 (the forward's without a mask) on large arrays whose length is a multiple of
+their vector; one Gaussian more (an odd length) takes the kernels that the other tests hold against the oracle,
+on the same values. Sizes: just above the backward's rule (48 MB of coefficients) with a last workgroup partly
+filled and lengths of 2 modulo 4, and just above the forward's (192 MB). Lower degrees and masked forwards of
+these sizes take the one-per-thread kernels either way.
 
 Bound: every value is a sum of at most 25 products per channel, taken in the same order; contraction may
 differ, so 2 x 25 x 2^-24 = 3e-6 of the sum of the terms' magnitudes, which is below 32 here; the position
@@ -22,6 +23,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("degree,dc,masked,mega", [
     (3, False, True, 48), (3, True, False, 48), (1, False, False, 48), (4, True, True, 48), (0, False, True, 48),
     (3, False, False, 192), (3, True, True, 192), (4, False, True, 192), (2, False, True, 192),
+    (3, True, False, 192), (4, False, False, 192), (4, True, False, 192), (4, False, False, 48),
 ])
 def test_wide_matches_single(degree, dc, masked, mega):
     bands = (degree + 1) ** 2 - (1 if dc else 0)

@@ -275,14 +275,20 @@ __global__ __launch_bounds__(kBlock) void sh_fwd_3kn_kernel(
 
 // [3, K, N] with V Gaussians per thread: every band row is read (and in the backward written) as V-wide
 // vectors, so that a wavefront keeps V times the bytes in flight. HBM-bound; backward alone, 1.5 M Gaussians
-// of degree 3: 143 -> 109 us (4.4 -> 5.8 TB/s), 300 k: 24 -> 20 us; but 400 k of degree 2 15 -> 17 us, so
-// coefficients of less than kVecBytes keep the one-per-thread kernel. The gradient rows bypass the caches
+// of degree 3: 143 -> 109 us (4.4 -> 5.8 TB/s), 300 k: 24 -> 20 us. From degree 3 only (kVecDegree), and from
+// kVecBytes of coefficients: lower degrees keep few enough loads a thread that vectors gain nothing, and the rows
+// they leave unread are zeroed faster by the other kernel (1 M Gaussians of 16 bands, two sets in turn, one per
+// thread against vectors: degree 0 29 us against 38, degree 2 of 9 bands 39 against 43; 300 k degree 2 15 against
+// 19). The gradient rows bypass the caches
 // (written once, read later). Coefficients that with their gradients outgrow the 256 MB last-level cache
 // (kStreamBytes) are read past it as well (NT), in the forward too, which gains nothing else from vectors:
 // both passes over three such sets in turn 217 -> 164 us (170 without), 1 M of degree 4 251 -> 171 (178); at
-// 115 MB 76 us against 67. Needs n a multiple of V and arrays aligned to the vectors (vec_ok); other calls
-// take the one-per-thread kernels. The values are computed as there, in the same order; only d_origin's
-// partial sums group other Gaussians.
+// 115 MB 76 us against 67. A masked forward keeps the other kernel: where the mask leaves runs out, the rows that
+// are read fit the cache that it reads past (2 M of degree 3, a quarter kept in runs of 4096: 25 us against 43;
+// half or a tenth kept at random 84 against 72). Needs n a multiple of V and arrays aligned to the vectors (vec_ok);
+// other calls take the one-per-thread kernels. The values are computed as there, in the same order; only
+// d_origin's partial sums group other Gaussians.
+constexpr int kVecDegree = 3;
 constexpr int64_t kVecBytes = 48ll << 20, kStreamBytes = 192ll << 20;
 
 template <bool NT, class T>
@@ -323,55 +329,35 @@ XSG_DEV void store3v(float* __restrict__ dst, const float (&v)[3 * V]) {
 template <int DEG, bool HAS_DC, int V>
 __global__ __launch_bounds__(kBlock) void sh_fwd_3kn_vec_kernel(
     int64_t n, int dim, const float* __restrict__ origin, const float* __restrict__ pos,
-    const float* __restrict__ coeffs, const float* __restrict__ dc, const uint32_t* __restrict__ mask,
-    int zero_masked, float* __restrict__ out) {
+    const float* __restrict__ coeffs, const float* __restrict__ dc, float* __restrict__ out) {
     typedef typename VecF<V>::type vf;
     constexpr int NY = (DEG + 1) * (DEG + 1);
     const int64_t i = V * ((int64_t)blockIdx.x * kBlock + threadIdx.x);
     if (i >= n) return;
-    bool ok[V], any = false, all = true;
+    float r[3 * V], p[3 * V];
+    load3v<V>(pos + 3 * i, p);
+    const f3 o = ld3(origin);
+    f3 dir[V];
+    float Y[V][NY];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-        ok[j] = mask_ok(mask, i + j);
-        any = any || ok[j];
-        all = all && ok[j];
+        const f3 diff = mk3(p[3 * j], p[3 * j + 1], p[3 * j + 2]) - o;
+        dir[j] = diff * (1.0f / sqrtf(dot(diff, diff)));
+        sh_basis<DEG>(dir[j], Y[j]);
     }
-    float r[3 * V];
 #pragma unroll
-    for (int j = 0; j < 3 * V; ++j) r[j] = 0.f;
-    if (any) {
-        float p[3 * V];
-        load3v<V>(pos + 3 * i, p);
-        const f3 o = ld3(origin);
-        f3 dir[V];
-        float Y[V][NY];
+    for (int c = 0; c < 3; ++c) {
+        vf b[NY];
 #pragma unroll
-        for (int j = 0; j < V; ++j) {
-            const f3 diff = mk3(p[3 * j], p[3 * j + 1], p[3 * j + 2]) - o;
-            dir[j] = diff * (1.0f / sqrtf(dot(diff, diff)));
-            sh_basis<DEG>(dir[j], Y[j]);
+        for (int k = 0; k < NY; ++k) {
+            const float* row = HAS_DC ? (k == 0 ? dc + (int64_t)c * n : coeffs + ((int64_t)c * dim + k - 1) * n)
+                                      : coeffs + ((int64_t)c * dim + k) * n;
+            b[k] = __builtin_nontemporal_load(reinterpret_cast<const vf*>(row + i));
         }
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            vf b[NY];
-#pragma unroll
-            for (int k = 0; k < NY; ++k) {
-                const float* row = HAS_DC ? (k == 0 ? dc + (int64_t)c * n : coeffs + ((int64_t)c * dim + k - 1) * n)
-                                          : coeffs + ((int64_t)c * dim + k) * n;
-                b[k] = __builtin_nontemporal_load(reinterpret_cast<const vf*>(row + i));
-            }
-#pragma unroll
-            for (int j = 0; j < V; ++j)
-                r[3 * j + c] = ok[j] ? sh_color<DEG>(dir[j], Y[j], [&](int k) { return b[k][j]; }) + 0.5f : 0.f;
-        }
+        for (int j = 0; j < V; ++j) r[3 * j + c] = sh_color<DEG>(dir[j], Y[j], [&](int k) { return b[k][j]; }) + 0.5f;
     }
-    if (all || zero_masked) {
-        store3v<V>(out + 3 * i, r);
-    } else {
-#pragma unroll
-        for (int j = 0; j < V; ++j)
-            if (ok[j]) st3(out + 3 * (i + j), mk3(r[3 * j], r[3 * j + 1], r[3 * j + 2]));
-    }
+    store3v<V>(out + 3 * i, r);
 }
 
 template <int DEG, bool HAS_DC, int V, bool NT>
@@ -645,10 +631,14 @@ constexpr int kBwdVec = 2;
 template <int DEG, bool DC>
 void launch_fwd(bool l3kn, dim3 g, hipStream_t s, int64_t n, int dim, const float* o, const float* p,
                 const float* c, const float* dc, const uint32_t* m, int zm, float* out) {
-    constexpr int V = kFwdVec<DEG>;
-    if (l3kn && 12 * dim * n >= kStreamBytes && vec_ok<V>(n, {p, c, dc, out}))
-        sh_fwd_3kn_vec_kernel<DEG, DC, V><<<xsg_blocks(n / V, kBlock), kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
-    else if (l3kn) sh_fwd_3kn_kernel<DEG, DC><<<g, kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
+    if constexpr (DEG >= kVecDegree) {
+        constexpr int V = kFwdVec<DEG>;
+        if (l3kn && !m && 12 * dim * n >= kStreamBytes && vec_ok<V>(n, {p, c, dc, out})) {
+            sh_fwd_3kn_vec_kernel<DEG, DC, V><<<xsg_blocks(n / V, kBlock), kBlock, 0, s>>>(n, dim, o, p, c, dc, out);
+            return;
+        }
+    }
+    if (l3kn) sh_fwd_3kn_kernel<DEG, DC><<<g, kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
     else sh_fwd_nk3_kernel<DEG, DC><<<g, kBlock, 0, s>>>(n, dim, o, p, c, dc, m, zm, out);
 }
 
@@ -657,14 +647,16 @@ template <int DEG, bool DC>
 unsigned launch_bwd(bool l3kn, dim3 g, hipStream_t s, int64_t n, int dim, const float* o, const float* p,
                 const float* c, const uint32_t* m, const float* dout, float* dcf, float* ddc, float* dp,
                 float* part) {
-    constexpr int V = kBwdVec;
-    if (l3kn && 12 * dim * n >= kVecBytes && vec_ok<V>(n, {p, c, dout, dcf, ddc, dp})) {
-        const unsigned nb = xsg_blocks(n / V, kBlock);
-        if (12 * dim * n >= kStreamBytes)
-            sh_bwd_3kn_vec_kernel<DEG, DC, V, true><<<nb, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
-        else
-            sh_bwd_3kn_vec_kernel<DEG, DC, V, false><<<nb, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
-        return nb;
+    if constexpr (DEG >= kVecDegree) {
+        constexpr int V = kBwdVec;
+        if (l3kn && 12 * dim * n >= kVecBytes && vec_ok<V>(n, {p, c, dout, dcf, ddc, dp})) {
+            const unsigned nb = xsg_blocks(n / V, kBlock);
+            if (12 * dim * n >= kStreamBytes)
+                sh_bwd_3kn_vec_kernel<DEG, DC, V, true><<<nb, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
+            else
+                sh_bwd_3kn_vec_kernel<DEG, DC, V, false><<<nb, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
+            return nb;
+        }
     }
     if (l3kn) sh_bwd_kernel<DEG, DC, true><<<g, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
     else sh_bwd_kernel<DEG, DC, false><<<g, kBlock, 0, s>>>(n, dim, o, p, c, m, dout, dcf, ddc, dp, part);
