@@ -242,7 +242,6 @@ __global__ __launch_bounds__(NT)
     __shared__ int32_t s_sbf[NSB];              // largest last id of each strip's pixels
     __shared__ uint64_t s_mask[NSB][NBW];       // [strip][staging wavefront]: Gaussians it evaluates
     __shared__ uint64_t s_high[NBW];
-    __shared__ uint64_t s_turn[3][NBW];         // one origin: the Gaussians' turns
     __shared__ __align__(16) float s_red[NWB][(K < 16 ? K : 16) * kRedRow];  // per wavefront: the gradient reduction
 
     const TileGrid& g = p.g;
@@ -390,7 +389,6 @@ __global__ __launch_bounds__(NT)
             const bool staged = tr < nb && idx >= range_start;
             StripCull cg;
             bool high = false;
-            Turn turn = {false, false, false};
             const int32_t fid = fid_next;
             if (tr < nb && idx - nb >= range_start) fid_next = p.flatten[idx - nb];
             float4* slot = s_slot + (tr < NB ? tr : 0) * kSlot4;
@@ -411,7 +409,6 @@ __global__ __launch_bounds__(NT)
                 }
                 if constexpr (FIXED) {
                     const RayFrame f = ray_frame(r0, r1, r2, at, o0, get_basis(s_frame));
-                    turn = f.turn;
                     slot[0] = make_float4(f.a1.x, f.a1.y, f.a1.z, f.D * f.D * -0.72134752f);
                     slot[1] = make_float4(f.a2.x, f.a2.y, f.a2.z, f.D);
                     slot[2] = make_float4(f.au.x, f.au.y, f.au.z, op);
@@ -452,10 +449,6 @@ __global__ __launch_bounds__(NT)
             {
                 const uint64_t m = __ballot(high);
                 if (lane == 0 && wave < nbw) s_high[wave] = m;
-            }
-            if constexpr (FIXED) {
-                const uint64_t mx = __ballot(turn.kx), my = __ballot(turn.ky), mn = __ballot(turn.neg);
-                if (lane == 0 && wave < nbw) { s_turn[0][wave] = mx; s_turn[1][wave] = my; s_turn[2][wave] = mn; }
             }
             if constexpr (NWB > 1)
                 for (int k = tr; k < nb * KT; k += (int)blockDim.x) s_tot[k] = 0.f;
@@ -611,9 +604,7 @@ __global__ __launch_bounds__(NT)
 #pragma unroll
                     for (int k = 0; k < 6; ++k) Q[k] = tot[G0 + 3 + k];
                     if constexpr (FIXED) {
-                        const uint64_t bit = 1ull << lane;
-                        const Turn turn = {(s_turn[0][w2] & bit) != 0, (s_turn[1][w2] & bit) != 0, (s_turn[2][w2] & bit) != 0};
-                        turn_back(r0, r1, r2, ld3(p.means + 3 * gid), o0, turn, vg, Q);
+                        turn_back(r0, r1, r2, ld3(p.means + 3 * gid), o0, vg, Q);
 #pragma unroll
                         for (int k = 0; k < 6; ++k) tot[G0 + 3 + k] = Q[k];
                     }

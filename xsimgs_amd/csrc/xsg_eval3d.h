@@ -42,18 +42,16 @@ XSG_DEV bool past_image(const TileGrid& g, int trow, int tcol) {
 }
 
 // Rows of M = S^-1 R^T from the raw quaternion (w, x, y, z) and activated scales: row i is column i
-// of R / s_i (utils.h:61-83 and eval3d_fwd.cu:92-107).
+// of R / s_i (utils.h:61-83 and eval3d_fwd.cu:92-107). Explicit roundings: see Turn.
 XSG_DEV void iscl_rot_rows(float4 q, f3 s, f3& r0, f3& r1, f3& r2) {
     float w = q.x, x = q.y, y = q.z, z = q.w;
-    const float inv = rsqrtf(x * x + y * y + z * z + w * w);
+    const float inv = rsqrtf(fmaf(w, w, fmaf(z, z, fmaf(y, y, x * x))));
     x *= inv; y *= inv; z *= inv; w *= inv;
-    const float x2 = x * x, y2 = y * y, z2 = z * z;
-    const float xy = x * y, xz = x * z, yz = y * z;
-    const float wx = w * x, wy = w * y, wz = w * z;
+    const float yz2 = fmaf(y, y, z * z), xz2 = fmaf(x, x, z * z), xy2 = fmaf(x, x, y * y), wx = w * x, wy = w * y, wz = w * z;
     const float i0 = 1.0f / s.x, i1 = 1.0f / s.y, i2 = 1.0f / s.z;
-    r0 = mk3(i0 * (1.f - 2.f * (y2 + z2)), i0 * (2.f * (xy + wz)), i0 * (2.f * (xz - wy)));
-    r1 = mk3(i1 * (2.f * (xy - wz)), i1 * (1.f - 2.f * (x2 + z2)), i1 * (2.f * (yz + wx)));
-    r2 = mk3(i2 * (2.f * (xz + wy)), i2 * (2.f * (yz - wx)), i2 * (1.f - 2.f * (x2 + y2)));
+    r0 = mk3(i0 * fmaf(-2.f, yz2, 1.f), i0 * (2.f * fmaf(x, y, wz)), i0 * (2.f * fmaf(x, z, -wy)));
+    r1 = mk3(i1 * (2.f * fmaf(x, y, -wz)), i1 * fmaf(-2.f, xz2, 1.f), i1 * (2.f * fmaf(y, z, wx)));
+    r2 = mk3(i2 * (2.f * fmaf(x, z, wy)), i2 * (2.f * fmaf(y, z, -wx)), i2 * fmaf(-2.f, xy2, 1.f));
 }
 
 XSG_DEV f3 sel3(bool c, f3 a, f3 b) { return mk3(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z); }
@@ -266,38 +264,47 @@ XSG_DEV void tile_bounds(TileFrame& f, const float4* boxes, int n_boxes, const f
     f.hx = hx; f.hy = hy; f.slack_o = __builtin_amdgcn_sqrtf(o); f.slack_t = t;
 }
 
-// One Gaussian's turned frame (rows in world space) and its affine rows (value, d/dx, d/dy).
-// The turn: which component of gro is the largest (x, else y, else z) and whether it is negative. Whoever turns
-// back takes it from here: another copy of the code may round a near tie the other way, and turn about another
-// axis.
+// The turn: the largest component of gro (kx: x, ky: y, else z), the components with that one (k) apart, and the
+// reflection I - beta n n^T, n = (ga, gb, vk), that sends gro to axis k. The backward derives it a second time, to
+// turn back: every rounding here and in the rows is therefore explicit (no sum that a compiler may contract one way
+// in one copy and another in the other), so that both copies take the same axis where components nearly tie.
 struct Turn {
-    bool kx, ky, neg;
+    bool kx, ky;
+    float gk, ga, gb, D, vk, beta;
 };
+XSG_DEV Turn turn_of(f3 r0, f3 r1, f3 r2, f3 v) {
+    auto dot1 = [](f3 a, f3 b) { return fmaf(a.z, b.z, fmaf(a.y, b.y, a.x * b.x)); };
+    const f3 g = mk3(dot1(r0, v), dot1(r1, v), dot1(r2, v));
+    const float ax = fabsf(g.x), ay = fabsf(g.y), az = fabsf(g.z);
+    Turn t;
+    t.kx = ax >= ay && ax >= az;
+    t.ky = !t.kx && ay >= az;
+    t.gk = t.kx ? g.x : t.ky ? g.y : g.z;
+    t.ga = t.kx ? g.y : g.x;
+    t.gb = (t.kx || t.ky) ? g.z : g.y;
+    t.D = __builtin_amdgcn_sqrtf(dot1(g, g));
+    t.vk = t.gk + copysignf(t.D, t.gk);
+    const float den = t.D * (t.D + fabsf(t.gk));
+    t.beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;  // at the Gaussian's centre any frame will do
+    return t;
+}
+
+// One Gaussian's turned frame (rows in world space) and its affine rows (value, d/dx, d/dy).
 struct RayFrame {
     f3 t1, t2, u;
     f3 a1, a2, au;
     float D;
-    Turn turn;
 };
 
 XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& bas) {
     const f3 v = o - mu;
-    const f3 g = rows_mul(r0, r1, r2, v);
-    const float ax = fabsf(g.x), ay = fabsf(g.y), az = fabsf(g.z);
-    const bool kx = ax >= ay && ax >= az, ky = !kx && ay >= az;
-    // rows and components with the largest one (k) apart
-    const f3 rk = sel3(kx, r0, sel3(ky, r1, r2)), ra = sel3(kx, r1, r0), rb = sel3(kx || ky, r2, r1);
-    const float gk = kx ? g.x : ky ? g.y : g.z, ga = kx ? g.y : g.x, gb = (kx || ky) ? g.z : g.y;
-    const float D = __builtin_amdgcn_sqrtf(dot(g, g));
-    const float vk = gk + copysignf(D, gk);
-    const float den = D * (D + fabsf(gk));
-    const float beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;  // at the Gaussian's centre any frame will do
-    const f3 w = ga * ra + gb * rb + vk * rk;
+    const Turn t = turn_of(r0, r1, r2, v);
+    const f3 rk = sel3(t.kx, r0, sel3(t.ky, r1, r2)), ra = sel3(t.kx, r1, r0), rb = sel3(t.kx || t.ky, r2, r1);
+    const f3 w = t.ga * ra + t.gb * rb + t.vk * rk;
     RayFrame f;
-    f.turn = Turn{kx, ky, signbit(gk)};
-    f.t1 = ra - (beta * ga) * w;
-    f.t2 = rb - (beta * gb) * w;
-    f.u = copysignf(1.0f, gk) * ((beta * vk) * w - rk);
+    f.t1 = ra - (t.beta * t.ga) * w;
+    f.t2 = rb - (t.beta * t.gb) * w;
+    f.u = copysignf(1.0f, t.gk) * ((t.beta * t.vk) * w - rk);
     const d3 v64 = d3{(double)o.x - (double)mu.x, (double)o.y - (double)mu.y, (double)o.z - (double)mu.z};
     const d3 q1 = to64(f.t1), q2 = to64(f.t2);
     const f3 bx = to32(bas.x), by = to32(bas.y), ba = to32(bas.a);
@@ -311,17 +318,12 @@ XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& ba
 }
 
 // A vector and a symmetric matrix (upper triangle, row-major) of the turned frame, turned back into the
-// Gaussian's own normalised frame; the rows, mean and origin are those ray_frame was given, the turn its own.
-XSG_DEV void turn_back(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, Turn turn, f3& v, float (&Q)[6]) {
-    const f3 g = rows_mul(r0, r1, r2, o - mu);
-    const bool kx = turn.kx, ky = turn.ky;
-    const float gk = kx ? g.x : ky ? g.y : g.z, ga = kx ? g.y : g.x, gb = (kx || ky) ? g.z : g.y;
-    const float D = __builtin_amdgcn_sqrtf(dot(g, g));
-    const float vk = gk + (turn.neg ? -D : D);
-    const float den = D * (D + fabsf(gk));
-    const float beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;
-    const float s = turn.neg ? 1.0f : -1.0f;  // u is s times the reflected row k
-    const f3 n = mk3(ga, gb, vk);
+// Gaussian's own normalised frame; the rows, mean and origin are those ray_frame was given.
+XSG_DEV void turn_back(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, f3& v, float (&Q)[6]) {
+    const Turn t = turn_of(r0, r1, r2, o - mu);
+    const bool kx = t.kx, ky = t.ky;
+    const float beta = t.beta, s = -copysignf(1.0f, t.gk);  // u is s times the reflected row k
+    const f3 n = mk3(t.ga, t.gb, t.vk);
     f3 w = mk3(v.x, v.y, s * v.z);
     w = w - (beta * dot(n, w)) * n;  // in the order (a, b, k)
     v = mk3(kx ? w.z : w.x, kx ? w.x : ky ? w.z : w.y, (kx || ky) ? w.y : w.z);
