@@ -1,5 +1,6 @@
 """The compositor's edge inputs against the float64 oracle: grids larger than the image, pixels without a ray,
-tiles of very wide rays, flat Gaussians seen from moving origins, and Gaussians whose turn is a near tie.
+tiles of very wide rays, flat Gaussians seen from moving origins, Gaussians whose turn is a near tie, and
+Gaussians at the camera or without an extent to speak of.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -309,3 +310,25 @@ def test_turn_of_near_ties():
             usual = size > np.quantile(size, 0.2)
             err = np.linalg.norm(got[name] - ref[name], axis=1)
             assert (err[usual] <= 1e-3 * size[usual]).all(), (name, int((err[usual] > 1e-3 * size[usual]).sum()), kw)
+
+
+@pytest.mark.parametrize("distance", [0.0, 1e-38, 1e-25, 3e-20, 1e-19, 3e-19, 1e-15])
+@pytest.mark.parametrize("scale", [0.1, 30.0])
+def test_gaussians_at_the_camera(distance, scale):
+    """A Gaussian that the camera sits in, down to distances whose squares float32 does not hold."""
+    W, H = 33, 20
+    s = _scene(W, H, (16, 16), n=6, seed=4)
+    g = np.random.default_rng(1)
+    s["ro"][...] = 0.0
+    d = g.normal(0, 1, (6, 3))
+    s["means"][:] = distance * d / np.linalg.norm(d, axis=1, keepdims=True)
+    s["scales"][:] = scale * g.uniform(0.5, 2.0, (6, 3))
+    out, work, T = _forward(s)
+    _check_images(out, _oracle_fwd(s), np.ones((H, W), bool))
+    v = _image_grads(W, H, 3)
+    ref = _oracle_bwd(s, np_(out[2]), np_(out[3]), v)
+    for kw in (dict(ray_grads=True), dict(ray_grads=False, pixels_per_lane=2), dict(ray_grads=False, pixels_per_lane=4)):
+        got = _backward(s, out, work, T, v, **kw)
+        for k in ("v_opacity", "v_colors", "v_means"):
+            assert np.linalg.norm(got[k] - ref[k]) <= 1e-3 * np.linalg.norm(ref[k]) + 1e-12, (k, kw)
+        assert all(np.isfinite(x).all() for x in got.values())

@@ -285,7 +285,8 @@ XSG_DEV Turn turn_of(f3 r0, f3 r1, f3 r2, f3 v) {
     t.D = __builtin_amdgcn_sqrtf(dot1(g, g));
     t.vk = t.gk + copysignf(t.D, t.gk);
     const float den = t.D * (t.D + fabsf(t.gk));
-    t.beta = den > 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;  // at the Gaussian's centre any frame will do
+    // at the Gaussian's centre any frame will do (and the reciprocals of smaller numbers are infinite)
+    t.beta = den > 1e-36f ? __builtin_amdgcn_rcpf(den) : 0.f;
     return t;
 }
 
@@ -309,7 +310,7 @@ XSG_DEV RayFrame ray_frame(f3 r0, f3 r1, f3 r2, f3 mu, f3 o, const TileBasis& ba
     const d3 q1 = to64(f.t1), q2 = to64(f.t2);
     const f3 bx = to32(bas.x), by = to32(bas.y), ba = to32(bas.a);
     const float vv = dot(v, v);
-    const float va = vv > 0.f ? dot(v, ba) * __builtin_amdgcn_rcpf(vv) : 0.f;
+    const float va = vv > 1e-37f && t.beta > 0.f ? dot(v, ba) * __builtin_amdgcn_rcpf(vv) : 0.f;
     f.a1 = mk3((float)(dot64(q1, bas.a) - (double)((float)dot64(q1, v64) * va)), dot(f.t1, bx), dot(f.t1, by));
     f.a2 = mk3((float)(dot64(q2, bas.a) - (double)((float)dot64(q2, v64) * va)), dot(f.t2, bx), dot(f.t2, by));
     f.au = mk3(dot(f.u, ba), dot(f.u, bx), dot(f.u, by));
