@@ -1,6 +1,6 @@
 """The compositor's edge inputs against the float64 oracle: grids larger than the image, pixels without a ray,
 tiles of very wide rays, flat Gaussians seen from moving origins, Gaussians whose turn is a near tie, and
-Gaussians at the camera or without an extent to speak of.
+Gaussians at the camera, and the launches whose LDS is sized for small workgroups.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -332,3 +332,20 @@ def test_gaussians_at_the_camera(distance, scale):
         for k in ("v_opacity", "v_colors", "v_means"):
             assert np.linalg.norm(got[k] - ref[k]) <= 1e-3 * np.linalg.norm(ref[k]) + 1e-12, (k, kw)
         assert all(np.isfinite(x).all() for x in got.values())
+
+
+@pytest.mark.parametrize("dynamic", [False, True])
+@pytest.mark.parametrize("tile,cdim", [((8, 8), 3), ((8, 8), 17), ((5, 7), 33), ((16, 8), 17), ((12, 10), 32), ((16, 8), 1),
+                                       ((13, 9), 33), ((32, 32), 16), ((32, 32), 17), ((32, 20), 9)])
+def test_small_and_large_workgroups(tile, cdim, dynamic):
+    """Tiles of one and two strips (one wavefront in the backward), whose workgroups have LDS of their own size, and
+    large tiles of many channels; lists that end inside, at and past a batch."""
+    W, H = 70, 45
+    v = _image_grads(W, H, cdim)
+    for n in (64, 130):
+        s = _scene(W, H, tile, n=n, cdim=cdim, dynamic=dynamic, seed=n)
+        out, work, T = _forward(s)
+        _check_images(out, _oracle_fwd(s), np.ones((H, W), bool))
+        ref = _oracle_bwd(s, np_(out[2]), np_(out[3]), v)
+        for ray_grads in ((True, False) if cdim <= 16 else (True,)):
+            _check_grads(_backward(s, out, work, T, v, ray_grads=ray_grads), ref)
