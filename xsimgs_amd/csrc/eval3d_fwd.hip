@@ -502,13 +502,23 @@ int launch_cdim(bool dyn, const Eval3dParams& p, hipStream_t s) {
     auto go = [&](auto count_c, auto dyn_c) {
         constexpr bool C = decltype(count_c)::value, D = decltype(dyn_c)::value;
         constexpr bool two = CDIM <= kFwdColorLdsMax;  // wider colours' sums fill the registers of one pixel
+        // large tiles: the general form takes its strips one at a time, which reads colours from HBM twice
+        // (32x32 tiles with motion: 16 channels 416 us against 333; but 9 channels 259 against 305)
+        constexpr int big = two && !(D && CDIM >= 16) ? 2 : 1;
         constexpr int U4 = CDIM <= 4 ? 4 : 1;
+        // With more than 16 channels in LDS a workgroup of one or two wavefronts takes arrays of its own size:
+        // those of four leave a compute unit four workgroups (17 channels, 37 KB; 1280x800 in 8x8 tiles: 370 us
+        // against 146)
+        constexpr bool sized = CDIM > 16 && CDIM <= kFwdColorLdsMax;
         if (tile_px > T)  // up to the reference's 1024 pixels (eval3d_fwd.cu:204-221)
-            eval3d_fwd_kernel<CDIM, D, two ? 2 : 1, 1, kMaxTilePixels / (two ? 2 : 1), C>
-                <<<n_blocks, two ? nt2 : nt1, 0, s>>>(p);
+            eval3d_fwd_kernel<CDIM, D, big, 1, kMaxTilePixels / big, C><<<n_blocks, big == 2 ? nt2 : nt1, 0, s>>>(p);
         else if (two && !D && strips % 2 == 0 && (int64_t)n_blocks * (nt2 / 64) >= kFwdTwoPixelWaves)
             eval3d_fwd_kernel<CDIM, false, two ? 2 : 1, 1, T / (two ? 2 : 1), C>
                 <<<n_blocks, two ? nt2 : nt1, 0, s>>>(p);
+        else if (sized && strips == 1)
+            eval3d_fwd_kernel<CDIM, D, 1, 1, sized ? T / 4 : T, C><<<n_blocks, nt1, 0, s>>>(p);
+        else if (sized && strips == 2)
+            eval3d_fwd_kernel<CDIM, D, 1, 1, sized ? T / 2 : T, C><<<n_blocks, nt1, 0, s>>>(p);
         else if ((int64_t)n_blocks * strips > kFwdDeepWaves)
             eval3d_fwd_kernel<CDIM, D, 1, 1, T, C><<<n_blocks, nt1, 0, s>>>(p);
         else
