@@ -242,6 +242,10 @@ __global__ __launch_bounds__(NT)
     __shared__ int32_t s_sbf[NSB];              // largest last id of each strip's pixels
     __shared__ uint64_t s_mask[NSB][NBW];       // [strip][staging wavefront]: Gaussians it evaluates
     __shared__ uint64_t s_high[NBW];
+    // where the totals go: the k-th one's array (in bytes from v_means) and its bytes per Gaussian. Looked up, the
+    // five arrays' addresses do not sit in scalar registers across the pair loops.
+    __shared__ int64_t s_dst[KT];
+    __shared__ uint32_t s_step[KT];
     __shared__ __align__(16) float s_red[NWB][(K < 16 ? K : 16) * kRedRow];  // per wavefront: the gradient reduction
 
     const TileGrid& g = p.g;
@@ -269,6 +273,27 @@ __global__ __launch_bounds__(NT)
         return q < bs && i < g.height && j < g.width ? (int64_t)cam * hw + (int64_t)i * g.width + j : -1;
     };
     auto pixel_of = [&](int h) { return pixel_at((wave * PX + h) * 64 + opaque(lane)); };
+    for (int k = tr; k < KT; k += (int)blockDim.x) {
+        const int kk = KO + k;
+        const float* dst;
+        int step = 3;
+        if (kk < CDIM) {  // colour gradients of camera cam start at cam * (n * CDIM - col_shift)
+            dst = p.v_colors + (int64_t)cam * (g.n * CDIM - p.col_shift) + kk;
+            step = CDIM;
+        } else if (kk < CDIM + 3) {
+            dst = p.v_means + (kk - CDIM);
+        } else if (kk < CDIM + 9) {
+            dst = p.v_mt + (kk - CDIM - 3);
+            step = 6;
+        } else if (kk == CDIM + 9) {
+            dst = p.v_opac;
+            step = 1;
+        } else {
+            dst = p.v_velocity + (kk - CDIM - 10);
+        }
+        s_dst[k] = reinterpret_cast<const char*>(dst) - reinterpret_cast<const char*>(p.v_means);
+        s_step[k] = 4 * step;
+    }
     // The left end of the tile's middle row, and that row's middle pixel (which stands in for those outside)
     const int64_t ps = (int64_t)cam * hw + (int64_t)min(trow * g.tile_h + g.tile_h / 2, g.height - 1) * g.width + tcol * g.tile_w;
     const int64_t pm = ps + min(g.tile_w / 2, g.width - 1 - tcol * g.tile_w);
@@ -306,34 +331,37 @@ __global__ __launch_bounds__(NT)
     const float rt0 = mid.t;
     const TileBasis basis = uniform_basis(tile_basis(mid.d, side));
     if (tr == 0) put_basis(s_frame, basis);
-    bool narrow = true, same = true;
+    bool same = true, some = false;
+    int bare = 0;  // strips
     float far2 = 0.f, late = 0.f;
     int32_t wave_bin_final = -1;
 #pragma unroll
     for (int h = 0; h < PX; ++h) {
         BwdPixel<CS>& q = px[h];
-        float ik = 0.f;
-        bool ray = true;
-        q.x = q.y = 0.f;
-        if (inside[h]) {
-            const f3 ro = ray_o[h], away = ro - o0;
-            const float rt = ray_t[h] - rt0;
-            ray = ray_xy(basis, ray_d[h], q.x, q.y, ik) && finite3(away) && isfinite(rt);
-            narrow = narrow && ray;
-            same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
-                   __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
-            far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
-            late = ray ? fmaxf(late, fabsf(rt)) : late;
-        }
-        const float4 box = strip_box(inside[h], ray, q.x, q.y);
-        if (lane == 0) s_box[wave * PX + h] = box;
-        q.v_t = ik;  // until the mode is known
+        const f3 away = ray_o[h] - o0;
+        const float rt = ray_t[h] - rt0;
+        float ik;
+        const bool ray = ray_xy(basis, ray_d[h], q.x, q.y, ik) && finite3(away) && isfinite(rt) && inside[h];
+        const float4 box = strip_box(ray, q.x, q.y);
+        same = same && (!ray || (__float_as_uint(ray_o[h].x) == __float_as_uint(o0.x) &&
+                                 __float_as_uint(ray_o[h].y) == __float_as_uint(o0.y) &&
+                                 __float_as_uint(ray_o[h].z) == __float_as_uint(o0.z)));
+        some = some || ray;
+        far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
+        late = ray ? fmaxf(late, fabsf(rt)) : late;
+        q.x = ray ? q.x : 0.f;
+        q.y = ray ? q.y : 0.f;
+        q.v_t = ray ? ik : 0.f;  // until the mode is known
+        if (__ballot(inside[h] && !ray) != 0) bare |= 1 << (wave * PX + h);
         const int m = wave_max(q.bin_final);
-        if (lane == 0) s_sbf[wave * PX + h] = m;
+        if (lane == 0) {
+            s_box[wave * PX + h] = box;
+            s_sbf[wave * PX + h] = m;
+        }
         wave_bin_final = max(wave_bin_final, m);
     }
     {
-        const int v = (__ballot(!narrow) == 0 ? 1 : 0) | (__ballot(!same) == 0 ? 2 : 0);
+        const int v = tile_vote(__ballot(!same) == 0, __ballot(some) != 0, bare);
         const float f = wave_max_f(far2), l = DYN ? wave_max_f(late) : 0.f;
         if (lane == 0) {
             s_vote[wave] = v;
@@ -343,28 +371,36 @@ __global__ __launch_bounds__(NT)
         }
     }
     __syncthreads();
-    int kind = 3, tile_max = -1;
+    int vote = -1, tile_max = -1;
     for (int k = 0; k < nwb; ++k) {
-        kind &= s_vote[k];
+        vote &= s_vote[k];
         tile_max = max(tile_max, s_max[k]);
     }
     if (tr == 0) tile_bounds(s_frame, s_box, nwb * PX, s_slack[0], s_slack[1], nwb);
     __syncthreads();
-    kind = __builtin_amdgcn_readfirstlane(kind);
-    const bool fixed = !DYN && kind == 3;
-    const bool rays = (kind & 1) != 0;  // every pixel has one
+    vote = __builtin_amdgcn_readfirstlane(vote);
+    const bool fixed = !DYN && (vote & (kVoteOneOrigin | kVoteNoRay)) == kVoteOneOrigin;
+    bare = bare_strips(vote);
 
     uint64_t n_eval = 0, n_contrib = 0;  // evaluated / composited pixel-pairs of the wave, when counting
-    const int32_t eff_end = min(range_end - 1, __builtin_amdgcn_readfirstlane(tile_max));
-    const int32_t n_eff = eff_end - range_start + 1;
-    const int num_batches = n_eff > 0 ? (n_eff + nb - 1) / nb : 0;
+    int32_t eff_end;
+    int num_batches;
+    auto list_up_to = [&](int32_t last) {  // the tile's list up to its pixels' largest last id
+        eff_end = min(range_end - 1, __builtin_amdgcn_readfirstlane(last));
+        const int32_t n_eff = eff_end - range_start + 1;
+        num_batches = n_eff > 0 ? (n_eff + nb - 1) / nb : 0;
+    };
+    list_up_to(tile_max);
 
     // the whole sweep is instantiated for both origin modes, so that neither carries the other's registers
     auto sweep = [&](auto fixed_c) {
         constexpr bool FIXED = decltype(fixed_c)::value;
 #pragma unroll
         for (int h = 0; h < PX; ++h) {
-            if constexpr (FIXED) px[h].v_d = -px[h].v_d * px[h].v_t;
+            if constexpr (FIXED) {
+                px[h].v_d = -px[h].v_d * px[h].v_t;
+                px[h].bin_final = px[h].v_t != 0.f ? px[h].bin_final : -1;
+            }
             px[h].v_t = 0.f;
         }
         f3 px_rd[FIXED ? 1 : PX], px_ro[FIXED ? 1 : PX];  // the pixels' rays and times
@@ -427,7 +463,7 @@ __global__ __launch_bounds__(NT)
                                            s_frame.slack_o + s_frame.slack_t * __builtin_amdgcn_sqrtf(dot(vel, vel)), s_frame);
                 }
                 // alphas may reach the clamp, or be no number
-                high = !(op <= kMaxAlpha) || cg.keep_all || !rays;
+                high = !(op <= kMaxAlpha) || cg.keep_all || (!FIXED && bare != 0);
                 if constexpr (CL > 0) {
                     const float* cp = p.colors + ((int64_t)fid * CDIM - (int64_t)cam * p.col_shift);
 #pragma unroll
@@ -442,7 +478,8 @@ __global__ __launch_bounds__(NT)
             // which strips evaluate this Gaussian: those with a pixel at or past it (last ids) that the
             // Gaussian can reach; one ballot per strip
             for (int k = 0; k < nwb * PX; ++k) {
-                const bool keep = staged && idx <= s_sbf[k] && strip_keep(s_box[k], cg);
+                const bool keep = staged && idx <= s_sbf[k] &&
+                                  ((!FIXED && ((bare >> k) & 1) != 0) || ((FIXED || !fixed) && strip_keep(s_box[k], cg)));
                 const uint64_t m = __ballot(keep);
                 if (lane == 0 && wave < nbw) s_mask[k][wave] = m;
             }
@@ -630,28 +667,52 @@ __global__ __launch_bounds__(NT)
                     const uint32_t gid = (uint32_t)(fid2 - (int64_t)cam * g.n);
 #pragma unroll
                     for (int ch = 0; ch < (KT + 15) / 16; ++ch) {
-                        const int kk = KO + 16 * ch + kk0;
-                        if (!on || kk >= K) continue;
-                        float* dst;
-                        if (kk < CDIM)  // colour gradients of camera cam start at cam * (n * CDIM - col_shift)
-                            dst = p.v_colors + (int64_t)cam * (g.n * CDIM - p.col_shift) + (uint64_t)gid * CDIM + kk;
-                        else if (kk < CDIM + 3) dst = p.v_means + (uint64_t)gid * 3 + (kk - CDIM);
-                        else if (kk < CDIM + 9) dst = p.v_mt + (uint64_t)gid * 6 + (kk - CDIM - 3);
-                        else if (kk == CDIM + 9) dst = p.v_opac + gid;
-                        else dst = p.v_velocity + (uint64_t)gid * 3 + (kk - CDIM - 10);
-                        unsafeAtomicAdd(dst, src[kk - KO]);
+                        const int k = 16 * ch + kk0;
+                        if (!on || k >= KT) continue;
+                        char* dst = reinterpret_cast<char*>(p.v_means) + s_dst[k] + (uint64_t)gid * s_step[k];
+                        unsafeAtomicAdd(reinterpret_cast<float*>(dst), src[k]);
                     }
                 }
             }
             __syncthreads();  // the slots are free for the next batch
         }
     };
-    if constexpr (DYN) {
-        sweep(std::false_type{});
-    } else {
-        if (fixed) sweep(std::true_type{});
-        else sweep(std::false_type{});
+    if constexpr (!DYN) {
+        if (fixed) {
+            sweep(std::true_type{});
+            if constexpr (RG) {  // in the tile's basis, and dL/dgrd times k
+                const TileBasis basis = get_basis(s_frame);
+                const f3 ba = to32(basis.a), bx = to32(basis.x), by = to32(basis.y);
+#pragma unroll
+                for (int h = 0; h < PX; ++h) {
+                    const int64_t pix = pixel_of(h);
+                    if (pix < 0) continue;
+                    float x, y, ik;
+                    ray_xy(basis, ld3(p.ray_d + 3 * pix), x, y, ik);
+                    f3 v = px[h].v_ro;
+                    px[h].v_ro = v.x * ba + v.y * bx + v.z * by;
+                    v = px[h].v_rd;
+                    px[h].v_rd = (px[h].bin_final >= 0 ? ik : 0.f) * (v.x * ba + v.y * bx + v.z * by);
+                }
+            }
+            if (bare != 0) {  // the pixels without a ray, left out above (last id -1), with their own last ids
+#pragma unroll
+                for (int h = 0; h < PX; ++h) {
+                    const int64_t pix = pixel_of(h);
+                    const bool in = pix >= 0 && px[h].bin_final < 0;
+                    px[h].bin_final = in ? p.last_ids[pix] : -1;
+                    px[h].v_d = in ? p.v_depth[pix] : 0.f;
+                    const int m = wave_max(px[h].bin_final);
+                    if (lane == 0) s_sbf[wave * PX + h] = m;
+                }
+                __syncthreads();
+                int32_t last = -1;
+                for (int k = 0; k < nwb * PX; ++k) last = max(last, s_sbf[k]);
+                list_up_to(last);
+            }
+        }
     }
+    if (DYN || !fixed || bare != 0) sweep(std::false_type{});
     if (COUNT && lane == 0) {  // one atomic per wave and counter
         atomicAdd(p.pair_counts, (unsigned long long)n_eval);
         atomicAdd(p.pair_counts + 1, (unsigned long long)n_contrib);
@@ -662,17 +723,8 @@ __global__ __launch_bounds__(NT)
             const int64_t pix = pixel_of(h);
             if (pix >= 0) {
                 if constexpr (RG) {
-                    f3 v_ro = px[h].v_ro, v_rd = px[h].v_rd;
-                    if (!DYN && fixed) {  // in the tile's basis, and dL/dgrd times k
-                        const TileBasis basis = get_basis(s_frame);
-                        float x, y, ik;
-                        ray_xy(basis, ld3(p.ray_d + 3 * pix), x, y, ik);
-                        const f3 ba = to32(basis.a), bx = to32(basis.x), by = to32(basis.y);
-                        v_ro = v_ro.x * ba + v_ro.y * bx + v_ro.z * by;
-                        v_rd = ik * (v_rd.x * ba + v_rd.y * bx + v_rd.z * by);
-                    }
-                    st3(p.v_ray_o + 3 * pix, v_ro);
-                    st3(p.v_ray_d + 3 * pix, v_rd);
+                    st3(p.v_ray_o + 3 * pix, px[h].v_ro);
+                    st3(p.v_ray_d + 3 * pix, px[h].v_rd);
                 }
                 if constexpr (DYN) p.v_time[pix] = px[h].v_t;
             }

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     __shared__ float4 s_col[C4 > 0 ? C4 : 1][NT + 1];
     __shared__ int32_t s_id[CL > 0 || CDIM == 0 ? 1 : NT + 1];
     __shared__ float4 s_box[NS];                        // the strips' boxes of (x, y)
-    __shared__ float s_ik[DYN ? 1 : PX][DYN ? 1 : NT];  // rays of one origin: each pixel's 1 / k
+    __shared__ float s_ik[DYN ? 1 : PX][DYN ? 1 : NT];  // each pixel's 1 / k, 0 without a ray
     __shared__ TileFrame s_frame;
     __shared__ float s_slack[2][NW];  // largest distance from the basis pixel's origin, and time from its own
     // [wavefront][staging wavefront]: the Gaussians it evaluates, and their number
@@ -161,37 +161,39 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     const float rt0 = mid.t;
     const TileBasis basis = uniform_basis(tile_basis(mid.d, side));
     if (tr == 0) put_basis(s_frame, basis);
-    bool narrow = true, same = true;
+    bool same = true, some = false, ray[PX];
+    int bare = 0;  // strips
     float far2 = 0.f, late = 0.f;
 #pragma unroll
     for (int h = 0; h < PX; ++h) {
-        float ik = 0.f;
-        bool ray = true;
-        px[h] = py[h] = 0.f;
-        if (inside[h]) {
-            const f3 ro = ray_o[h], away = ro - o0;
-            const float rt = ray_t[h] - rt0;
-            ray = ray_xy(basis, ray_d[h], px[h], py[h], ik) && finite3(away) && isfinite(rt);
-            same = same && __float_as_uint(ro.x) == __float_as_uint(o0.x) &&
-                   __float_as_uint(ro.y) == __float_as_uint(o0.y) && __float_as_uint(ro.z) == __float_as_uint(o0.z);
-            far2 = ray ? fmaxf(far2, dot(away, away)) : far2;
-            late = ray ? fmaxf(late, fabsf(rt)) : late;
-            narrow = narrow && ray;
-        }
-        const float4 box = strip_box(inside[h], ray, px[h], py[h]);
+        const f3 away = ray_o[h] - o0;
+        const float rt = ray_t[h] - rt0;
+        float ik;
+        ray[h] = ray_xy(basis, ray_d[h], px[h], py[h], ik) && finite3(away) && isfinite(rt) && inside[h];
+        const float4 box = strip_box(ray[h], px[h], py[h]);
+        same = same && (!ray[h] || (__float_as_uint(ray_o[h].x) == __float_as_uint(o0.x) &&
+                                    __float_as_uint(ray_o[h].y) == __float_as_uint(o0.y) &&
+                                    __float_as_uint(ray_o[h].z) == __float_as_uint(o0.z)));
+        some = some || ray[h];
+        far2 = ray[h] ? fmaxf(far2, dot(away, away)) : far2;
+        late = ray[h] ? fmaxf(late, fabsf(rt)) : late;
+        px[h] = ray[h] ? px[h] : 0.f;
+        py[h] = ray[h] ? py[h] : 0.f;
+        if (__ballot(inside[h] && !ray[h]) != 0) bare |= 1 << (wave * PX + h);
         if (lane == 0) s_box[wave * PX + h] = box;
-        if constexpr (!DYN) s_ik[h][tr] = ik;
+        if constexpr (!DYN) s_ik[h][tr] = ray[h] ? ik : 0.f;
     }
     {
-        const int v = (__ballot(!narrow) == 0 ? 1 : 0) | (__ballot(!same) == 0 ? 2 : 0);
+        const int v = tile_vote(__ballot(!same) == 0, __ballot(some) != 0, bare);
         if (lane == 0) s_vote[wave] = v;
         const float f = wave_max_f(far2), l = DYN ? wave_max_f(late) : 0.f;
         if (lane == 0) { s_slack[0][wave] = f; s_slack[1][wave] = l; }
     }
     __syncthreads();
-    const int kind = votes();
-    // one origin (as float32 values) and ordinary rays: the pairs in the turned frame's affine form
-    const bool fixed = !DYN && kind == 3;
+    const int vote = votes();
+    // one origin (as float32 values): the pairs in the turned frame's affine form
+    const bool fixed = !DYN && (vote & (kVoteOneOrigin | kVoteNoRay)) == kVoteOneOrigin;
+    bare = bare_strips(vote);
     if (tr == 0) tile_bounds(s_frame, s_box, nw * PX, s_slack[0], s_slack[1], nw);
     __syncthreads();
 
@@ -205,8 +207,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
 #pragma unroll
     for (int h = 0; h < PX; ++h) {
         T[h] = 1.f; depth[h] = 0.f; cur_idx[h] = 0;
-        thr[h] = inside[h] ? kOpen : __builtin_inff();
-        open[h] = __ballot(inside[h]);
+        const bool in = fixed ? ray[h] : inside[h];
+        thr[h] = in ? kOpen : __builtin_inff();
+        open[h] = __ballot(in);
 #pragma unroll
         for (int k = 0; k < CS; ++k) acc[h][k] = 0.f;
     }
@@ -274,7 +277,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
                 if (staged) {
 #pragma unroll 1
                     for (int h = 0; h < PX; ++h)
-                        keep = keep || strip_keep(s_box[k * PX + h], cg);
+                        keep = keep || (!FIXED && ((bare >> (k * PX + h)) & 1) != 0) ||
+                               ((FIXED || !fixed) && strip_keep(s_box[k * PX + h], cg));
                 }
                 const uint64_t m = __ballot(keep);
                 const int cnt = (int)__popcll(m);
@@ -453,12 +457,25 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
             raw = load_raw(staged_at(b));
         }
     };
-    if constexpr (DYN) {
-        sweep(std::false_type{});
-    } else {
-        if (fixed) sweep(std::true_type{});
-        else sweep(std::false_type{});
+    if constexpr (!DYN) {
+        if (fixed) {
+            sweep(std::true_type{});
+#pragma unroll
+            for (int h = 0; h < PX; ++h) depth[h] = -depth[h] * s_ik[h][tr];
+            if (bare != 0) {  // the pixels without a ray, which took nothing yet
+                __syncthreads();
+#pragma unroll
+                for (int h = 0; h < PX; ++h) {
+                    const bool in = pixel_of(h) >= 0 && s_ik[h][tr] == 0.f;
+                    thr[h] = in ? kOpen : __builtin_inff();
+                    open[h] = __ballot(in);
+                }
+                if (num_batches > 0 && staged_at(0)) fid_next = p.flatten[(uint32_t)range_start + (uint32_t)tr];
+                raw = load_raw(num_batches > 0 && staged_at(0));
+            }
+        }
     }
+    if (DYN || !fixed || bare != 0) sweep(std::false_type{});
     if (COUNT && lane == 0) {  // one atomic per wave and counter
         atomicAdd(p.pair_counts, (unsigned long long)n_eval);
         atomicAdd(p.pair_counts + 1, (unsigned long long)n_contrib);
@@ -468,9 +485,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
         const int64_t pix = pixel_of(h);
         if (pix >= 0) {
             p.out_alpha[pix] = 1.0f - T[h];
-            float dep = depth[h];
-            if constexpr (!DYN) dep = fixed ? -dep * s_ik[h][tr] : dep;
-            p.out_depth[pix] = dep;
+            p.out_depth[pix] = depth[h];
 #pragma unroll
             for (int k = 0; k < CDIM; ++k) p.out_rgb[pix * CDIM + k] = acc[h][k];
             p.out_last[pix] = cur_idx[h];

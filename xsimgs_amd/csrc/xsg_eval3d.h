@@ -2,10 +2,11 @@
 //
 // One workgroup per (camera, tile). The tile's pixels form strips of 64 consecutive ones (row-major); a
 // wavefront owns one or more whole strips, one pixel of each per lane. Gaussians of the tile's depth-sorted
-// list are staged in LDS in batches. Tiles whose rays all start at one origin, are rays (finite, not zero) and
-// run within 84 degrees of the tile's middle one work in a turned frame and affine ray coordinates (below; a
-// block vote decides, and a static pinhole, fisheye or spherical camera's tiles pass unless they are masked or
-// span half the sphere); the others with the rows of M = S^-1 R^T, as the reference does per pair.
+// list are staged in LDS in batches. Where all rays of a tile start at one origin and run within 84 degrees of the
+// middle one, the tile is swept in a turned frame and affine ray coordinates (below; a block vote decides, and the
+// tiles of a static pinhole, fisheye or spherical camera pass unless they span half the sphere); else with the rows
+// of M = S^-1 R^T, as the reference does per pair. Pixels without such a ray (masked ones, say) do not hold the
+// others back: they are swept by themselves, a second time through the list, in the second form.
 #pragma once
 #include "xsg_common.h"
 
@@ -235,25 +236,31 @@ XSG_DEV bool ray_xy(const TileBasis& b, f3 d, float& x, float& y, float& inv_k) 
     return regular_ray(d) && k > 0.0 && k * k > 0.01 * dot64(v, v);
 }
 
-// The box of (x, y) that 64 pixels' rays fill: centre and half extents (hx < 0: no pixel; infinite: a pixel
-// whose ray gives no (x, y), or no ray at all, which any Gaussian may reach: that strip alone is then not
-// culled). Whether there is a pixel is never told from the coordinates, which are NaN then.
-XSG_DEV float4 strip_box(bool inside, bool ray, float x, float y) {
+// The box of (x, y) that the rays of a strip's 64 pixels fill: centre and half extents (hx < 0: no pixel has a
+// ray). A pixel whose ray gives no (x, y), or is none at all, is a bare one: it is in no box, any Gaussian may reach
+// it, and its strip is kept whole where it is evaluated.
+XSG_DEV float4 strip_box(bool ray, float x, float y) {
     const float big = __builtin_inff();
-    const float x0 = wave_min_f(inside ? x : big), x1 = wave_max_f(inside ? x : -big);
-    const float y0 = wave_min_f(inside ? y : big), y1 = wave_max_f(inside ? y : -big);
-    if (__ballot(inside) == 0) return make_float4(0.f, 0.f, -1.f, -1.f);
-    if (__ballot(inside && !ray) != 0) return make_float4(0.f, 0.f, big, big);
+    const float x0 = wave_min_f(ray ? x : big), x1 = wave_max_f(ray ? x : -big);
+    const float y0 = wave_min_f(ray ? y : big), y1 = wave_max_f(ray ? y : -big);
+    if (__ballot(ray) == 0) return make_float4(0.f, 0.f, -1.f, -1.f);
     return make_float4(0.5f * (x0 + x1), 0.5f * (y0 + y1), 0.500001f * (x1 - x0) + 1.2e-7f * (1.f + fabsf(x0) + fabsf(x1)),
                        0.500001f * (y1 - y0) + 1.2e-7f * (1.f + fabsf(y0) + fabsf(y1)));
 }
 
-// The tile's largest |x| and |y| (of the strips that are culled) and its slack (strip_cull), from its strips' and
-// wavefronts'.
+// A wavefront's vote on its tile (the tile's is their conjunction): the pixels that have a ray share the basis
+// pixel's origin; no pixel has one. And in the complement (so that the conjunction is their union), from bit 8 on,
+// the strips with bare pixels.
+constexpr int kVoteOneOrigin = 1, kVoteNoRay = 2;
+XSG_DEV int tile_vote(bool one_origin, bool has_ray, int bare_strips) {
+    return (one_origin ? kVoteOneOrigin : 0) | (has_ray ? 0 : kVoteNoRay) | (~bare_strips << 8);
+}
+XSG_DEV int bare_strips(int vote) { return (~vote >> 8) & 0xffff; }
+
+// The tile's largest |x| and |y| and its slack (strip_cull), from its strips' and wavefronts'.
 XSG_DEV void tile_bounds(TileFrame& f, const float4* boxes, int n_boxes, const float* far2, const float* late, int nw) {
     float hx = 0.f, hy = 0.f, o = 0.f, t = 0.f;
     for (int k = 0; k < n_boxes; ++k) {
-        if (!(boxes[k].z < __builtin_inff())) continue;
         hx = fmaxf(hx, fabsf(boxes[k].x) + boxes[k].z);
         hy = fmaxf(hy, fabsf(boxes[k].y) + boxes[k].w);
     }
@@ -422,7 +429,7 @@ XSG_DEV StripCull strip_cull(const RayFrame& f, const CullInput& in, float hx, f
                   det_err * fabsf(c.xg)) * 1.0002f;
     c.ey = aid * (reach * __builtin_amdgcn_sqrtf(f.a1.y * f.a1.y + f.a2.y * f.a2.y) + 4e-6f * (fabsf(ny0) + fabsf(ny1)) +
                   det_err * fabsf(c.yg)) * 1.0002f;
-    c.ex = drop_all ? -__builtin_inff() : c.ex;  // out of every finite box
+    c.ex = drop_all ? -__builtin_inff() : c.ex;  // out of every box
     return c;
 }
 
@@ -447,8 +454,7 @@ XSG_DEV StripCull strip_cull_moving(f3 r0, f3 r1, f3 r2, f3 at, f3 s, CullInput 
     return strip_cull(f, in, tile.hx, tile.hy);
 }
 
-// True unless no pixel of the strip can take the Gaussian (every comparison fails on a NaN, so none of them
-// drops a Gaussian from an infinite box).
+// True unless no pixel in the strip's box can take the Gaussian (every comparison fails on a NaN).
 XSG_DEV bool strip_keep(float4 box, const StripCull& c) {
     const float b1 = fabsf(fmaf(box.y, c.a1.z, fmaf(box.x, c.a1.y, c.a1.x))) - fabsf(c.a1.y) * box.z - fabsf(c.a1.z) * box.w;
     const float b2 = fabsf(fmaf(box.y, c.a2.z, fmaf(box.x, c.a2.y, c.a2.x))) - fabsf(c.a2.y) * box.z - fabsf(c.a2.z) * box.w;
