@@ -62,7 +62,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     __shared__ float4 s_op[OP_IN_COL ? 1 : NT + 1];  // opacity, when no colour slot has room
     __shared__ float4 s_vel[DYN ? NT + 1 : 1];
     __shared__ float4 s_col[C4 > 0 ? C4 : 1][NT + 1];
-    __shared__ int32_t s_id[CL > 0 || CDIM == 0 ? 1 : NT + 1];
+    __shared__ int32_t s_id[CL > 0 || CDIM == 0 ? 1 : NT];
+    static_assert(U == 1 || CL > 0 || CDIM == 0, "the lists' filling has no colours in HBM");
     __shared__ float4 s_box[NS];                        // the strips' boxes of (x, y)
     __shared__ float s_ik[DYN ? 1 : PX][DYN ? 1 : NT];  // each pixel's 1 / k, 0 without a ray
     __shared__ TileFrame s_frame;
@@ -139,7 +140,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
         if constexpr (!OP_IN_COL) s_op[NT] = make_float4(0.f, 0.f, 0.f, 0.f);
         if constexpr (DYN) s_vel[NT] = make_float4(0.f, 0.f, 0.f, 0.f);
         for (int k4 = 0; k4 < C4; ++k4) s_col[k4][NT] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (CL == 0 && CDIM > 0) s_id[NT] = 0;
     }
     // The pixels' rays and times, loaded before the basis pixel's is looked at (their latencies overlap)
     f3 ray_o[PX], ray_d[PX];
