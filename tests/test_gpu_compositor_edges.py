@@ -1,6 +1,7 @@
 """The compositor's edge inputs against the float64 oracle: grids larger than the image, pixels without a ray,
 tiles of very wide rays, flat Gaussians seen from moving origins, Gaussians whose turn is a near tie, and
-Gaussians at the camera, and the launches whose LDS is sized for small workgroups.
+Gaussians at the camera, Gaussians of no or infinite extent or that are no numbers, and
+the launches whose LDS is sized for small workgroups.
 
 Every tile lists the same Gaussians in depth order. Bounds are the suite's: 1e-4 absolute on the renders of all
 but one pixel in ten thousand, 1e-3 of an array's norm on gradients.
@@ -179,6 +180,7 @@ def test_pixels_without_a_ray(kind, moving, dynamic, where, tile):
     W, H = 97, 81
     s = _scene(W, H, tile, moving=moving, dynamic=dynamic)
     bad = _spoil(s, where, kind)
+    s["opac"][::7] = 0.002  # (below the threshold, but not at 0.999)
     out, work, T = _forward(s)
     ref = _oracle_fwd(s)
     _check_images(out, ref, ~bad)
@@ -349,3 +351,18 @@ def test_small_and_large_workgroups(tile, cdim, dynamic):
         ref = _oracle_bwd(s, np_(out[2]), np_(out[3]), v)
         for ray_grads in ((True, False) if cdim <= 16 else (True,)):
             _check_grads(_backward(s, out, work, T, v, ray_grads=ray_grads), ref)
+
+
+@pytest.mark.parametrize("moving,dynamic", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("what,value", [("opac", np.nan), ("opac", np.inf), ("means", np.nan), ("means", np.inf),
+                                        ("quats", 0.0), ("quats", np.nan), ("scales", 0.0), ("scales", np.nan),
+                                        ("scales", np.inf)])
+def test_gaussians_that_are_no_numbers(what, value, moving, dynamic):
+    """They reach the alpha test as they are: an alpha that is no number is 0.999, and a Gaussian of infinite extent
+    has its opacity everywhere. (Depths are not compared: such a Gaussian's is no number.)"""
+    W, H = 50, 37
+    s = _scene(W, H, (16, 16), n=40, moving=moving, dynamic=dynamic)
+    s["opac"] *= np.float32(0.3)
+    s[what][17] = value
+    out, work, T = _forward(s)
+    _check_images(out, _oracle_fwd(s), np.ones((H, W), bool), depth=False)
