@@ -10,8 +10,8 @@
 //    scale gradients once per Gaussian by the epilogue: quat_scale_to_preci_half_vjp
 //    (utils.h:232-263) is linear in dL/dM, so the sum of per-pair vjps equals the vjp of the sum,
 //    and the scale gradient is -Q_ii / s_i;
-//  * tiles whose rays share one origin work in the forward's turned frame and affine form (xsg_eval3d.h); Q and the mean's gradient are turned back once per
-//    Gaussian and batch;
+//  * tiles whose rays share one origin work in the forward's turned frame and affine form (xsg_eval3d.h); Q and
+//    the mean's gradient are turned back once per Gaussian and batch;
 //  * per-pair gradients are summed over the 64 lanes of a wavefront through LDS and the totals left in the
 //    Gaussian's own staging slot; after a batch one lane per Gaussian finishes them (the turn, M^T, the
 //    opacity) and the atomics add 16 components of four Gaussians per instruction;
@@ -21,7 +21,7 @@
 //  * divisions in the per-pair math are reciprocal-multiplies (v_rcp_f32, 1 ulp).
 //
 // Bound by VALU issue. The whole op against per-pair M^T products and atomics per Gaussian and wavefront, in the
-// unturned frame: 1920x1080, 1 M Gaussians 422 -> 343 us; six cameras of 1600x900 1675 -> 1240; moving origins
+// unturned frame: 1920x1080, 1 M Gaussians 422 -> 333-352 us; six cameras of 1600x900 1675 -> 1240; moving origins
 // 459 -> 312; 32 channels at 640x480 445 -> 316; 2048x128 lidar 189 -> 172.
 //
 // This header holds the kernel template and its per-CDIM launcher; eval3d_bwd_g*.hip instantiate the

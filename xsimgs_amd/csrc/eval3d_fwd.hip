@@ -15,8 +15,8 @@
 //    is a pixel that no alpha reaches (its threshold becomes infinite). Running out is tested once for the
 //    U Gaussians and resolved apart, which each pixel does at most once.
 // The whole op against one pixel per lane, a bit scan per Gaussian and every tile evaluated as M (ro - mu), M rd:
-// 1920x1080, 1 M Gaussians 240 -> 171-190 us; six cameras of 1600x900 886 -> 655; 1237x701 115 -> 85; 2048x128 lidar
-// 72 -> 49; 256x256 63 -> 25; 32 channels at 640x480 170 -> 88; moving origins, which keep that form, 154 -> 154.
+// 1920x1080, 1 M Gaussians 240 -> 188-197 us; six cameras of 1600x900 886 -> 655-716; 1237x701 115 -> 85; 2048x128
+// lidar 72 -> 49-54; 256x256 63 -> 25; 32 channels at 640x480 170 -> 88; moving origins, which keep that form, 154 -> 154.
 #include <type_traits>
 
 #include "xsg_eval3d.h"
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kFwdWaves<CD
     __syncthreads();
 
     // A pixel takes a pair when alpha > thr: the largest float below 1/255 while the pixel is open, then
-    // infinity (also outside the image).
+    // infinity (also outside the image, and in the other form's sweep).
     constexpr float kOpen = 0.00392156839370728f;  // 1.f / 255.f less one ulp
     float T[PX], depth[PX], thr[PX], acc[PX][CS];
     uint64_t open[PX];  // the wavefront's open pixels

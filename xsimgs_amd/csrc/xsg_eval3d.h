@@ -381,12 +381,6 @@ struct StripCull {
     bool keep_all;
 };
 
-// d_lim: sqrt(2 ln(255 op)) through log2; + 3e-3 covers the rounding of log, exp, the product and the compare.
-XSG_DEV float reach_of(float op) {
-    const float l2 = 2.f * 0.69314718f * __builtin_amdgcn_logf(fmaxf(255.f * op, 1.f));
-    return __builtin_amdgcn_sqrtf(l2) * 1.0001f + 3e-3f;
-}
-
 // What of a Gaussian the test needs beside its frame, taken before it (its inputs then end there).
 struct CullInput {
     float lim;       // d_lim
